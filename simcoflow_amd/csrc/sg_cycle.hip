@@ -23,9 +23,13 @@ namespace {
 constexpr int NTB = 256;
 
 constexpr int TAIL_MAX = 1024;   // levels with at most this many points run in the tail kernel
-constexpr int TAIL_THREADS = 1024;
+// threads of the tail, a 2x2 block of its first level each: 256 for up to 256
+// blocks, as on a level of 32 x 32 -- one wavefront per SIMD, so that a
+// thread's couplings, weights and vectors fit its registers in FP64 too -- and
+// 512 for the longer or odd levels, none of which has more blocks
+constexpr int TAIL_NT = 256, TAIL_NT_MAX = 512;
 constexpr int MAX_TAIL = 10;
-constexpr size_t TAIL_LDS_MAX = 150 * 1024;  // of the 160 KB of LDS a workgroup can hold
+constexpr size_t TAIL_LDS_MAX = 150 * 1024;  // of the tail levels' operators, vectors and weights
 
 struct Slots {
     double* part;
@@ -748,15 +752,31 @@ void launch_up5(bool semi, hipStream_t s, Dims F, OpV<T> A, const V* b, const T*
 }
 
 // ---------------------------------------------------------------------------
-// tail: the V-cycle on levels lt..nlev-1 in one workgroup, all of it in LDS
-// (compact layout cd: ld = ni+1; the arrays of a level follow each other)
+// tail: levels lt..nlev-1 in one workgroup.
+//
+// Nothing here is bound by bytes or operations: a V-cycle of these levels is a
+// chain of some twenty passes, each waiting for the neighbours' values of the
+// one before, so a pass costs an LDS round trip, its arithmetic's latency and a
+// barrier.  The split keeps that chain short:
+//   level 0 (lt)   a thread owns a 2x2 block of cells, its couplings and
+//                  values in registers; LDS carries only what neighbours read.
+//                  The block is one point of level 1,
+//   level 1        which the same thread owns: the restricted residual and the
+//                  prolongation's weights never leave its registers;
+//   levels 2..     small enough for one wavefront as a rule, which then runs
+//                  them without barriers while the others wait at one.
+// A colour pass reads the other colour from one array and writes its own to
+// another, so one barrier ends it.  Sums keep one order of terms and cells,
+// which is the level's and not that of the threads.  At 32 x 32 points, 4 inner
+// iterations, FP64 / FP32: 39 / 39 us; with a thread per cell, every level in
+// LDS and sixteen wavefronts at each barrier, 53 / 56 us.
 enum { TA_D = 0, TA_E, TA_N, TA_NE, TA_NW, TA_X, TA_B, TA_R, TA_COUNT };
 
 template <typename T>
 struct TailLevel {
     Dims d;   // global layout
-    Dims cd;  // LDS layout
-    int base;  // LDS offset (elements) of this level's TA_COUNT arrays
+    Dims cd;  // LDS layout of a level >= 2
+    int base;  // LDS offset (elements) of such a level's TA_COUNT arrays
     int wbase; // LDS offset of its 9 prolongation-weight arrays (next level's cd)
     int sh;    // thread k of a pass takes cell (k & (2^sh - 1), k >> sh), 2^sh >= ni
     OpV<T> A;
@@ -772,11 +792,12 @@ struct TailArgs {
     const double* inv;  // dense inverse of the coarsest operator (FP64 in both precisions)
     const int* on; // the PCG's convergence flag (the cycle runs while *on), or null
     int krylov;    // inner flexible-CG iterations on the first tail level (0: one V-cycle)
-    int pbase;     // LDS offset of the inner iteration's direction vector
-    int invbase;   // LDS offset (in T) of the staged FP64 dense inverse, 8-byte aligned
+    int ld0, x0, x1;  // level 0's arrays XA, XB: element (i, j) at (j + 1) * ld0 + i + 1
+    int ld1, y0, y1;  // level 1's arrays YA, YB, likewise
+    int lin;          // three level 0 vectors in linear order (inner iterations)
 };
 
-// offset of cell (i,j) in a level's LDS arrays (compact layout, 32-bit)
+// offset of cell (i,j) in the LDS arrays of a level >= 2 (compact layout)
 __device__ inline int toff(const Dims& D, int i, int j) { return (j + 2) * D.ld + i; }
 
 template <typename T>
@@ -784,11 +805,28 @@ __device__ inline T* tarr(T* lds, const TailLevel<T>& L, int k) {
     return lds + L.base + (size_t)k * L.cd.alloc_elems();
 }
 
-// One colour pass of the smoother, double-buffered: the cells of colour
-// `col` get (b + sum of couplings * src) / d, the others keep src; every
-// cell is written to dst, so one barrier ends the pass (same-colour diagonal
-// couplings read src, i.e. Jacobi-wise).  zero_start: src = 0.
-template <typename T>
+// ends a pass of the threads that run levels >= 2: the whole workgroup, or one
+// wavefront, whose LDS accesses are in order and only must not be moved
+template <bool WAVE>
+__device__ __forceinline__ void tail_sync() {
+    if (WAVE) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+// threads that run them
+template <bool WAVE>
+__device__ __forceinline__ int tail_threads() {
+    return WAVE ? 64 : (int)blockDim.x;
+}
+
+// One colour pass on a level >= 2, double-buffered: the cells of colour `col`
+// get (b + sum of couplings * src) / d, the others keep src; every cell is
+// written to dst, so one barrier ends the pass (same-colour diagonal couplings
+// read src, i.e. Jacobi-wise).  zero_start: src = 0.
+template <bool WAVE, typename T>
 __device__ void tail_pass(T* lds, const TailLevel<T>& L, const T* src, T* dst, int col, bool zero_start) {
     const Dims& D = L.cd;
     const int ld = D.ld;
@@ -799,7 +837,7 @@ __device__ void tail_pass(T* lds, const TailLevel<T>& L, const T* src, T* dst, i
     const T* nw = tarr(lds, L, TA_NW);
     const T* b = tarr(lds, L, TA_B);
     const int mask = (1 << L.sh) - 1;
-    for (int k = threadIdx.x; k < (D.nj << L.sh); k += TAIL_THREADS) {
+    for (int k = threadIdx.x; k < (D.nj << L.sh); k += tail_threads<WAVE>()) {
         const int i = k & mask, j = k >> L.sh;
         if (i >= D.ni) continue;
         const int p = toff(D, i, j);
@@ -817,158 +855,63 @@ __device__ void tail_pass(T* lds, const TailLevel<T>& L, const T* src, T* dst, i
         }
         dst[p] = v;
     }
-    __syncthreads();
+    tail_sync<WAVE>();
 }
 
-// The first tail level's couplings of the cell a thread owns in every pass,
-// held in registers for the whole kernel (used when each thread has at most
-// one cell of that level: (nj << sh) <= TAIL_THREADS)
-template <typename T>
-struct OwnRow {
-    bool own;  // the thread has a cell
-    int col;   // its colour, (i + j) & 1
-    int p;     // its LDS offset
-    T d, ew, ee, ns, nn, ne, nesw, nw, nwse;  // d[p], e[p-1], e[p], n[p-ld], n[p], ne[p], ne[p-ld-1], nw[p], nw[p-ld+1]
-};
-
-template <typename T>
-__device__ OwnRow<T> own_row(T* lds, const TailLevel<T>& L) {
-    OwnRow<T> R{};
-    const Dims& D = L.cd;
-    const int k = threadIdx.x, i = k & ((1 << L.sh) - 1), j = k >> L.sh;
-    R.own = k < (D.nj << L.sh) && i < D.ni;
-    if (!R.own) return R;
-    const int ld = D.ld, p = toff(D, i, j);
-    const T* d = tarr(lds, L, TA_D);
-    const T* e = tarr(lds, L, TA_E);
-    const T* nn = tarr(lds, L, TA_N);
-    const T* ne = tarr(lds, L, TA_NE);
-    const T* nw = tarr(lds, L, TA_NW);
-    R.col = (i + j) & 1;
-    R.p = p;
-    R.d = d[p];
-    R.ew = e[p - 1];
-    R.ee = e[p];
-    R.ns = nn[p - ld];
-    R.nn = nn[p];
-    R.ne = ne[p];
-    R.nesw = ne[p - ld - 1];
-    R.nw = nw[p];
-    R.nwse = nw[p - ld + 1];
-    return R;
+// dense solve on the coarsest level in FP64 (in both precisions): four threads
+// per row of the inverse in LDS, B(q) and X(row) the level's values.  Run by
+// the first wavefront.
+template <typename BF, typename XF>
+__device__ __forceinline__ void tail_dense(const double* inv, int n, BF B, XF X) {
+    const int row = threadIdx.x >> 2, quarter = threadIdx.x & 3;
+    double s = 0.0;
+    if (row < n)
+        for (int q = quarter; q < n; q += 4) s += inv[row * n + q] * (double)B(q);
+    s += __shfl_xor(s, 1, 64);
+    s += __shfl_xor(s, 2, 64);
+    if (row < n && quarter == 0) X(row, s);
 }
 
-// tail_pass on the first level with the couplings from registers (same
-// terms in the same order)
-template <typename T>
-__device__ void tail_pass_own(T* lds, const TailLevel<T>& L, const OwnRow<T>& R, const T* src, T* dst, int col,
-                              bool zero_start) {
-    if (R.own) {
-        const int ld = L.cd.ld, p = R.p;
-        const T* b = tarr(lds, L, TA_B);
-        T v = zero_start ? T(0) : src[p];
-        if (R.col == col) {
-            const T dd = R.d;
-            if (zero_start) {
-                v = dd > T(0) ? b[p] / dd : T(0);
-            } else {
-                const T s = R.ew * src[p - 1] + R.ee * src[p + 1] + R.ns * src[p - ld] + R.nn * src[p + ld] +
-                            R.ne * src[p + ld + 1] + R.nesw * src[p - ld - 1] + R.nw * src[p + ld - 1] +
-                            R.nwse * src[p - ld + 1];
-                v = dd > T(0) ? (b[p] + s) / dd : T(0);
-            }
-        }
-        dst[p] = v;
-    }
-    __syncthreads();
-}
-
-// stage operators, weights and the first level's b into LDS
-template <typename T>
-__device__ void tail_stage(T* lds, const TailArgs<T>& a) {
-    const int tid = threadIdx.x;
-    // stage operators, weights and the first level's b
-    for (int l = 0; l < a.n; ++l) {
-        const TailLevel<T>& L = a.L[l];
-        const int n = L.d.ni * L.d.nj;
-        const bool nine = L.A.cNE != nullptr;
-        for (int k = tid; k < n; k += TAIL_THREADS) {
-            const int i = k % L.d.ni, j = k / L.d.ni;
-            const size_t g = L.d.off(i, j), c = L.cd.off(i, j);
-            tarr(lds, L, TA_D)[c] = L.A.diag[g];
-            tarr(lds, L, TA_E)[c] = L.A.cE[g];
-            tarr(lds, L, TA_N)[c] = L.A.cN[g];
-            tarr(lds, L, TA_NE)[c] = nine ? L.A.cNE[g] : T(0);
-            tarr(lds, L, TA_NW)[c] = nine ? L.A.cNW[g] : T(0);
-            if (l == 0) tarr(lds, L, TA_B)[c] = L.b[g];
-        }
-        if (l + 1 < a.n) {
-            const TailLevel<T>& Cl = a.L[l + 1];
-            const int nc = Cl.d.ni * Cl.d.nj;
-            for (int k = tid; k < nc; k += TAIL_THREADS) {
-                const int I = k % Cl.d.ni, J = k / Cl.d.ni;
-                const size_t g = Cl.d.off(I, J), c = Cl.cd.off(I, J);
-#pragma unroll
-                for (int m = 0; m < 9; ++m) lds[L.wbase + (size_t)m * Cl.cd.alloc_elems() + c] = L.P.w[m][g];
-            }
-        }
-    }
-}
-
-// One V-cycle over the tail levels: level 0's TA_B -> level 0's TA_R.  On
+// V-cycle on the levels 2.. from level 2's TA_B to its TA_R (a.n > 2).  On
 // every level the smoothed x ends in TA_R; TA_X holds the first pass and then
 // the residual that is restricted.
-// With `regs`, level 0 takes its couplings from R (each thread's cell).
-template <typename T>
-__device__ void tail_vcycle(T* lds, const TailArgs<T>& a, const OwnRow<T>& R, bool regs) {
+template <bool WAVE, typename T>
+__device__ void tail_lower(T* lds, const TailArgs<T>& a, const double* inv) {
+    const int NTH = tail_threads<WAVE>();
     const int tid = threadIdx.x;
     const int last = a.n - 1;
-    for (int l = 0; l < last; ++l) {
+    for (int l = 2; l < last; ++l) {
         const TailLevel<T>& L = a.L[l];
         const TailLevel<T>& Cl = a.L[l + 1];
         const Dims& D = L.cd;
         const int ld = D.ld;
-        T* xa = tarr(lds, L, TA_X);
-        T* xb = tarr(lds, L, TA_R);
+        T* r = tarr(lds, L, TA_X);
+        T* x = tarr(lds, L, TA_R);
         const T* b = tarr(lds, L, TA_B);
-        const T* x = xb;
-        T* r = xa;
-        if (l == 0 && regs) {
-            tail_pass_own<T>(lds, L, R, nullptr, xa, 0, true);
-            tail_pass_own<T>(lds, L, R, xa, xb, 1, false);
-            if (R.own) {
-                const int p = R.p;
-                const T s = R.ew * x[p - 1] + R.ee * x[p + 1] + R.ns * x[p - ld] + R.nn * x[p + ld] +
-                            R.ne * x[p + ld + 1] + R.nesw * x[p - ld - 1] + R.nw * x[p + ld - 1] +
-                            R.nwse * x[p - ld + 1];
-                r[p] = b[p] - R.d * x[p] + s;
-            }
-        } else {
-            tail_pass<T>(lds, L, nullptr, xa, 0, true);
-            tail_pass<T>(lds, L, xa, xb, 1, false);
-            const T* d = tarr(lds, L, TA_D);
-            const T* e = tarr(lds, L, TA_E);
-            const T* nn = tarr(lds, L, TA_N);
-            const T* ne = tarr(lds, L, TA_NE);
-            const T* nw = tarr(lds, L, TA_NW);
-            const int mask = (1 << L.sh) - 1;
-            for (int k = tid; k < (D.nj << L.sh); k += TAIL_THREADS) {
-                const int i = k & mask;
-                if (i >= D.ni) continue;
-                const int p = toff(D, i, k >> L.sh);
-                const T s = e[p - 1] * x[p - 1] + e[p] * x[p + 1] + nn[p - ld] * x[p - ld] + nn[p] * x[p + ld] +
-                            ne[p] * x[p + ld + 1] + ne[p - ld - 1] * x[p - ld - 1] + nw[p] * x[p + ld - 1] +
-                            nw[p - ld + 1] * x[p - ld + 1];
-                r[p] = b[p] - d[p] * x[p] + s;
-            }
+        tail_pass<WAVE, T>(lds, L, nullptr, r, 0, true);
+        tail_pass<WAVE, T>(lds, L, r, x, 1, false);
+        const T* d = tarr(lds, L, TA_D);
+        const T* e = tarr(lds, L, TA_E);
+        const T* nn = tarr(lds, L, TA_N);
+        const T* ne = tarr(lds, L, TA_NE);
+        const T* nw = tarr(lds, L, TA_NW);
+        const int mask = (1 << L.sh) - 1;
+        for (int k = tid; k < (D.nj << L.sh); k += NTH) {
+            const int i = k & mask;
+            if (i >= D.ni) continue;
+            const int p = toff(D, i, k >> L.sh);
+            const T s = e[p - 1] * x[p - 1] + e[p] * x[p + 1] + nn[p - ld] * x[p - ld] + nn[p] * x[p + ld] +
+                        ne[p] * x[p + ld + 1] + ne[p - ld - 1] * x[p - ld - 1] + nw[p] * x[p + ld - 1] +
+                        nw[p - ld + 1] * x[p - ld + 1];
+            r[p] = b[p] - d[p] * x[p] + s;
         }
-        __syncthreads();
+        tail_sync<WAVE>();
         T* bc = tarr(lds, Cl, TA_B);
         const Dims& Cd = Cl.cd;
         const int ws = (int)Cd.alloc_elems(), cld = Cd.ld;
         const T* w0 = lds + L.wbase;
         const int cmask = (1 << Cl.sh) - 1;
-        for (int k = tid; k < (Cd.nj << Cl.sh); k += TAIL_THREADS) {
+        for (int k = tid; k < (Cd.nj << Cl.sh); k += NTH) {
             const int I = k & cmask, J = k >> Cl.sh;
             if (I >= Cd.ni) continue;
             const int c = toff(Cd, I, J), f = toff(D, 2 * I, 2 * J);
@@ -980,27 +923,19 @@ __device__ void tail_vcycle(T* lds, const TailArgs<T>& a, const OwnRow<T>& R, bo
                  w[W_NE * ws - cld - 1] * r[f - ld - 1];
             bc[c] = s;
         }
-        __syncthreads();
+        tail_sync<WAVE>();
     }
     {
-        // dense solve on the coarsest level in FP64 (in both precisions):
-        // four threads per row, the inverse staged in LDS
         const TailLevel<T>& L = a.L[last];
         const Dims& D = L.cd;
-        const int n = D.ni * D.nj;
         const T* b = tarr(lds, L, TA_B);
-        const double* inv = reinterpret_cast<const double*>(lds + a.invbase);
         T* x = tarr(lds, L, TA_R);
-        const int row = tid >> 2, quarter = tid & 3;
-        double s = 0.0;
-        if (row < n)
-            for (int q = quarter; q < n; q += 4) s += inv[row * n + q] * (double)b[D.off(q % D.ni, q / D.ni)];
-        s += __shfl_xor(s, 1, 64);
-        s += __shfl_xor(s, 2, 64);
-        if (row < n && quarter == 0) x[D.off(row % D.ni, row / D.ni)] = (T)s;
-        __syncthreads();
+        if (tid < 64)
+            tail_dense(inv, D.ni * D.nj, [&](int q) { return b[D.off(q % D.ni, q / D.ni)]; },
+                       [&](int q, double v) { x[D.off(q % D.ni, q / D.ni)] = (T)v; });
+        tail_sync<WAVE>();
     }
-    for (int l = last - 1; l >= 0; --l) {
+    for (int l = last - 1; l >= 2; --l) {
         const TailLevel<T>& L = a.L[l];
         const TailLevel<T>& Cl = a.L[l + 1];
         const Dims& D = L.cd;
@@ -1011,7 +946,7 @@ __device__ void tail_vcycle(T* lds, const TailArgs<T>& a, const OwnRow<T>& R, bo
         T* xa = tarr(lds, L, TA_X);
         T* xb = tarr(lds, L, TA_R);
         const int mask = (1 << L.sh) - 1;
-        for (int k = tid; k < (D.nj << L.sh); k += TAIL_THREADS) {
+        for (int k = tid; k < (D.nj << L.sh); k += NTH) {
             const int i = k & mask, j = k >> L.sh;
             if (i >= D.ni) continue;
             const int c = toff(Cd, i >> 1, j >> 1);
@@ -1025,34 +960,386 @@ __device__ void tail_vcycle(T* lds, const TailArgs<T>& a, const OwnRow<T>& R, bo
                      w[W_NE * ws] * ec[c + cld + 1];
             xb[toff(D, i, j)] += v;
         }
-        __syncthreads();
-        if (l == 0 && regs) {
-            tail_pass_own<T>(lds, L, R, xb, xa, 1, false);
-            tail_pass_own<T>(lds, L, R, xa, xb, 0, false);
-        } else {
-            tail_pass<T>(lds, L, xb, xa, 1, false);
-            tail_pass<T>(lds, L, xa, xb, 0, false);
-        }
+        tail_sync<WAVE>();
+        tail_pass<WAVE, T>(lds, L, xb, xa, 1, false);
+        tail_pass<WAVE, T>(lds, L, xa, xb, 0, false);
     }
 }
 
-// Sum of v over the workgroup, returned to every thread (part: 16 slots of
-// LDS per value, not reused before a barrier)
-template <int NV>
-__device__ inline void tail_allreduce(double (&v)[NV], double (*part)[NV]) {
+// A row's couplings in registers (all zero for a point outside the level)
+template <typename T>
+__device__ __forceinline__ Row9<T> tail_row(const TailLevel<T>& L, int i, int j) {
+    if (i < L.d.ni && j < L.d.nj) return load_row9(L.A, L.d.off(i, j), L.d.ld);
+    return Row9<T>{};
+}
+// sums of couplings * neighbours, one order everywhere; axis_sum where the
+// diagonal neighbours are zero
+template <typename T>
+__device__ __forceinline__ T axis_sum(const Row9<T>& r, T w, T e, T s, T n) {
+    return r.w * w + r.e * e + r.s * s + r.n * n;
+}
+template <typename T>
+__device__ __forceinline__ T full_sum(const Row9<T>& r, T w, T e, T s, T n, T ne, T sw, T nw, T se) {
+    return r.w * w + r.e * e + r.s * s + r.n * n + r.ne * ne + r.sw * sw + r.nw * nw + r.se * se;
+}
+// Gauss-Seidel value of a row from its right-hand side and that sum
+template <typename T>
+__device__ __forceinline__ T relaxed(const Row9<T>& r, T b, T s) {
+    return r.d > T(0) ? (b + s) / r.d : T(0);
+}
+// x + v with v rounded first (a correction is one value whatever its number of terms)
+template <typename T>
+__device__ __forceinline__ T corrected(T x, T v) {
+#pragma clang fp contract(off)
+    return x + v;
+}
+
+// The restriction's weights of coarse point (I, J), in restrict_point's order,
+// and the prolongation's to the 2x2 cells of that point
+template <typename T>
+__device__ __forceinline__ void restrict_weights(const Dims& C, const Prol<T>& P, int I, int J, T (&rw)[9]) {
+    T* const* w = P.w;
+    const size_t c = C.off(I, J), cw = C.off(I - 1, J), cs = C.off(I, J - 1), csw = C.off(I - 1, J - 1);
+    rw[0] = w[W_INJ][c];
+    rw[1] = w[W_XW][c];
+    rw[2] = w[W_XE][cw];
+    rw[3] = w[W_YS][c];
+    rw[4] = w[W_YN][cs];
+    rw[5] = w[W_SW][c];
+    rw[6] = w[W_SE][cw];
+    rw[7] = w[W_NW][cs];
+    rw[8] = w[W_NE][csw];
+}
+
+// Sums over the cells of level 0 in their linear order, returned to every
+// thread: F(t, v) gives cell t's terms; 64 cells reduce as a wavefront's
+// butterfly, the groups of 64 add up in order.  (The order is the level's, not
+// the threads' that own its blocks.)  part is not reused before another barrier.
+constexpr int TAIL_GROUPS = TAIL_MAX / 64;
+template <int NT, int NV, typename CellF>
+__device__ __forceinline__ void tail_allreduce(CellF F, double (&sum)[NV], double (*part)[NV]) {
+    double v[TAIL_MAX / NT][NV];
+#pragma unroll
+    for (int g = 0; g < TAIL_MAX / NT; ++g) F((int)threadIdx.x + g * NT, v[g]);
 #pragma unroll
     for (int k = 0; k < NV; ++k)
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) v[k] += __shfl_xor(v[k], m, 64);
+        for (int m = 32; m >= 1; m >>= 1)
+#pragma unroll
+            for (int g = 0; g < TAIL_MAX / NT; ++g) v[g][k] += __shfl_xor(v[g][k], m, 64);
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
-        for (int k = 0; k < NV; ++k) part[threadIdx.x >> 6][k] = v[k];
+        for (int g = 0; g < TAIL_MAX / NT; ++g)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) part[(threadIdx.x >> 6) + g * (NT / 64)][k] = v[g][k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         double s = 0.0;
-        for (int w = 0; w < TAIL_THREADS / 64; ++w) s += part[w][k];
-        v[k] = s;
+#pragma unroll
+        for (int w = 0; w < TAIL_GROUPS; ++w) s += part[w][k];
+        sum[k] = s;
+    }
+}
+
+// A thread's part of the levels
+template <typename T>
+struct TailOwn {
+    // level 0: cells 0 (2I,2J), 1 (2I+1,2J), 2 (2I,2J+1), 3 (2I+1,2J+1); 0 and 3 are red
+    Row9<T> r[4];
+    int p;     // LDS offset of cell 0
+    bool own;  // the thread has a block, and point (I, J) of level 1
+    // level 1
+    Row9<T> r1;
+    int p1;
+    bool red1;
+    T rw[9], pw[9];  // restriction from the block and prolongation to it
+    T pw1[4];        // its prolongation from level 2: from point e2, the one east of it, north, north-east
+    int par1, e2;    // parity bits (x, y) of the point
+    // level 2
+    Row9<T> r2;
+    int c2, f2;  // LDS offset of the thread's point (-1: none), and of the level 1 point on it
+    bool red2;
+    T rw2[9];
+};
+
+// cells around a block: south row, west and east columns, north row
+template <typename T>
+struct Ring12 {
+    T s0, s1, s2, s3, w0, w1, e0, e1, n0, n1, n2, n3;
+};
+template <typename T>
+__device__ __forceinline__ Ring12<T> ring(const T* x, int ld) {
+    return Ring12<T>{x[-ld - 1], x[-ld],    x[-ld + 1],    x[-ld + 2], x[-1],         x[ld - 1],
+                     x[2],       x[ld + 2], x[2 * ld - 1], x[2 * ld],  x[2 * ld + 1], x[2 * ld + 2]};
+}
+// sum of couplings * x over the neighbours of each cell of the block
+template <typename T>
+__device__ __forceinline__ void block_sums(const TailOwn<T>& O, const Ring12<T>& g, const T (&x)[4], T (&s)[4]) {
+    s[0] = full_sum(O.r[0], g.w0, x[1], g.s1, x[2], x[3], g.s0, g.w1, g.s2);
+    s[1] = full_sum(O.r[1], x[0], g.e0, g.s2, x[3], g.e1, g.s1, x[2], g.s3);
+    s[2] = full_sum(O.r[2], g.w1, x[3], x[0], g.n1, g.n2, g.w0, g.n0, x[1]);
+    s[3] = full_sum(O.r[3], x[2], g.e1, x[1], g.n2, g.n3, x[0], g.n1, g.e0);
+}
+// the sum over a point's eight neighbours in an array
+template <typename T>
+__device__ __forceinline__ T point_sum(const Row9<T>& r, const T* x, int ld) {
+    return full_sum(r, x[-1], x[1], x[-ld], x[ld], x[ld + 1], x[-ld - 1], x[ld - 1], x[1 - ld]);
+}
+
+// Level 2 and the dense solve below it on one wavefront, a point a lane (a.n =
+// 4): from the right-hand side b2 to the level's TA_R
+template <typename T>
+__device__ __forceinline__ void tail_level2(T* lds, const TailArgs<T>& a, const TailOwn<T>& O, const double* inv,
+                                            T b2) {
+    const TailLevel<T>& L = a.L[2];
+    const TailLevel<T>& C = a.L[3];
+    const Dims& D = L.cd;
+    const Dims& Dc = C.cd;
+    const int ld = D.ld;
+    const bool own = O.c2 >= 0;
+    const int c2 = own ? O.c2 : 0;
+    T* xa = tarr(lds, L, TA_X) + c2;
+    T* xb = tarr(lds, L, TA_R) + c2;
+    T* ec = tarr(lds, C, TA_R);
+    T x2 = T(0);
+    if (O.red2) x2 = relaxed(O.r2, b2, T(0));
+    if (own) xa[0] = x2;
+    tail_sync<true>();
+    if (own && !O.red2) {
+        x2 = relaxed(O.r2, b2, axis_sum(O.r2, xa[-1], xa[1], xa[-ld], xa[ld]));
+        xa[0] = x2;
+    }
+    tail_sync<true>();
+    if (own) xb[0] = b2 - O.r2.d * x2 + point_sum(O.r2, xa, ld);
+    tail_sync<true>();
+    const int ws = (int)Dc.alloc_elems(), cld = Dc.ld;
+    const int k3 = threadIdx.x;
+    if (k3 < Dc.ni * Dc.nj) {
+        const int I = k3 % Dc.ni, J = k3 / Dc.ni;
+        const T* r = tarr(lds, L, TA_R) + toff(D, 2 * I, 2 * J);
+        const T* w = lds + L.wbase + toff(Dc, I, J);
+        T s = w[W_INJ * ws] * r[0];
+        s += w[W_XW * ws] * r[1] + w[W_XE * ws - 1] * r[-1];
+        s += w[W_YS * ws] * r[ld] + w[W_YN * ws - cld] * r[-ld];
+        s += w[W_SW * ws] * r[ld + 1] + w[W_SE * ws - 1] * r[ld - 1] + w[W_NW * ws - cld] * r[1 - ld] +
+             w[W_NE * ws - cld - 1] * r[-ld - 1];
+        tarr(lds, C, TA_B)[toff(Dc, I, J)] = s;
+    }
+    tail_sync<true>();
+    const T* b3 = tarr(lds, C, TA_B);
+    tail_dense(inv, Dc.ni * Dc.nj, [&](int q) { return b3[toff(Dc, q % Dc.ni, q / Dc.ni)]; },
+               [&](int q, double v) { ec[toff(Dc, q % Dc.ni, q / Dc.ni)] = (T)v; });
+    tail_sync<true>();
+    if (own) {
+        const int i = threadIdx.x % D.ni, j = threadIdx.x / D.ni;
+        const int c = toff(Dc, i >> 1, j >> 1);
+        const T* w = lds + L.wbase + c;
+        const T* e = ec + c;
+        const int pi = i & 1, pj = j & 1;
+        T v;
+        if (!pi && !pj) v = w[W_INJ * ws] * e[0];
+        else if (pi && !pj) v = w[W_XW * ws] * e[0] + w[W_XE * ws] * e[1];
+        else if (!pi && pj) v = w[W_YS * ws] * e[0] + w[W_YN * ws] * e[cld];
+        else v = w[W_SW * ws] * e[0] + w[W_SE * ws] * e[1] + w[W_NW * ws] * e[cld] + w[W_NE * ws] * e[cld + 1];
+        x2 = corrected(x2, v);
+        xa[0] = x2;
+    }
+    tail_sync<true>();
+    T dne = T(0), dsw = T(0), dnw = T(0), dse = T(0);
+    if (own) {
+        dne = xa[ld + 1];
+        dsw = xa[-ld - 1];
+        dnw = xa[ld - 1];
+        dse = xa[1 - ld];
+        if (!O.red2) {
+            x2 = relaxed(O.r2, b2, full_sum(O.r2, xa[-1], xa[1], xa[-ld], xa[ld], dne, dsw, dnw, dse));
+            xb[0] = x2;
+        }
+    }
+    tail_sync<true>();
+    if (own && O.red2)
+        xb[0] = relaxed(O.r2, b2, full_sum(O.r2, xb[-1], xb[1], xb[-ld], xb[ld], dne, dsw, dnw, dse));
+    tail_sync<true>();
+}
+
+// One V-cycle over the tail levels: b -> x on the thread's block.  lower: how
+// the levels 2.. run (TAIL_LOWER_*).
+enum { TAIL_LOWER_ALL = 0, TAIL_LOWER_WAVE, TAIL_LOWER_OWN };
+template <typename T>
+__device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const TailOwn<T>& O, const double* inv,
+                                            int lower, const T (&b)[4], T (&x)[4]) {
+    const int tid = threadIdx.x;
+    T* XA = lds + a.x0;
+    T* XB = lds + a.x1;
+    T* YA = lds + a.y0;
+    T* YB = lds + a.y1;
+    const int ld = a.ld0, ld1 = a.ld1;
+    T* xa = XA + O.p;
+    T* xb = XB + O.p;
+    if (a.n == 1) {
+        // the first tail level is the coarsest
+        const Dims& D = a.L[0].d;
+        if (O.own) {
+            xa[0] = b[0];
+            xa[1] = b[1];
+            xa[ld] = b[2];
+            xa[ld + 1] = b[3];
+        }
+        __syncthreads();
+        auto at = [&](int q) { return (q / D.ni + 1) * ld + q % D.ni + 1; };
+        if (tid < 64)
+            tail_dense(inv, D.ni * D.nj, [&](int q) { return XA[at(q)]; }, [&](int q, double v) { XB[at(q)] = (T)v; });
+        __syncthreads();
+        if (O.own) {
+            x[0] = xb[0];
+            x[1] = xb[1];
+            x[2] = xb[ld];
+            x[3] = xb[ld + 1];
+        }
+        return;
+    }
+    // level 0 down: red from zero, black, residual
+    x[0] = relaxed(O.r[0], b[0], T(0));
+    x[3] = relaxed(O.r[3], b[3], T(0));
+    if (O.own) {
+        xa[0] = x[0];
+        xa[ld + 1] = x[3];
+    }
+    __syncthreads();
+    if (O.own) {
+        // the black cells were zero, so only red neighbours count
+        x[1] = relaxed(O.r[1], b[1], axis_sum(O.r[1], x[0], xa[2], xa[1 - ld], x[3]));
+        x[2] = relaxed(O.r[2], b[2], axis_sum(O.r[2], xa[ld - 1], x[3], x[0], xa[2 * ld]));
+        xa[1] = x[1];
+        xa[ld] = x[2];
+    }
+    __syncthreads();
+    T r[4] = {T(0), T(0), T(0), T(0)};
+    if (O.own) {
+        T s[4];
+        block_sums(O, ring(xa, ld), x, s);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = b[k] - O.r[k].d * x[k] + s[k];
+        xb[0] = r[0];
+        xb[1] = r[1];
+        xb[ld] = r[2];
+        xb[ld + 1] = r[3];
+    }
+    __syncthreads();
+    // level 1: its right-hand side, then the same
+    T b1 = T(0), x1 = T(0);
+    T* ya = YA + O.p1;
+    T* yb = YB + O.p1;
+    if (O.own) {
+        b1 = O.rw[0] * r[0];
+        b1 += O.rw[1] * r[1] + O.rw[2] * xb[-1];
+        b1 += O.rw[3] * r[2] + O.rw[4] * xb[-ld];
+        b1 += O.rw[5] * r[3] + O.rw[6] * xb[ld - 1] + O.rw[7] * xb[1 - ld] + O.rw[8] * xb[-ld - 1];
+    }
+    if (a.n == 2) {
+        const Dims& D = a.L[1].d;
+        if (O.own) ya[0] = b1;
+        __syncthreads();
+        auto at = [&](int q) { return (q / D.ni + 1) * ld1 + q % D.ni + 1; };
+        if (tid < 64)
+            tail_dense(inv, D.ni * D.nj, [&](int q) { return YA[at(q)]; }, [&](int q, double v) { YB[at(q)] = (T)v; });
+        __syncthreads();
+    } else {
+        if (O.red1) x1 = relaxed(O.r1, b1, T(0));
+        if (O.own) ya[0] = x1;
+        __syncthreads();
+        if (O.own && !O.red1) {
+            x1 = relaxed(O.r1, b1, axis_sum(O.r1, ya[-1], ya[1], ya[-ld1], ya[ld1]));
+            ya[0] = x1;
+        }
+        __syncthreads();
+        if (O.own) yb[0] = b1 - O.r1.d * x1 + point_sum(O.r1, ya, ld1);
+        __syncthreads();
+        // levels 2..
+        const TailLevel<T>& L2 = a.L[2];
+        T b2 = T(0);
+        if (O.c2 >= 0) {
+            const T* f = YB + O.f2;
+            b2 = O.rw2[0] * f[0];
+            b2 += O.rw2[1] * f[1] + O.rw2[2] * f[-1];
+            b2 += O.rw2[3] * f[ld1] + O.rw2[4] * f[-ld1];
+            b2 += O.rw2[5] * f[ld1 + 1] + O.rw2[6] * f[ld1 - 1] + O.rw2[7] * f[1 - ld1] + O.rw2[8] * f[-ld1 - 1];
+            if (lower != TAIL_LOWER_OWN) tarr(lds, L2, TA_B)[O.c2] = b2;
+        }
+        if (lower == TAIL_LOWER_OWN) {
+            if (tid < 64) tail_level2(lds, a, O, inv, b2);
+            __syncthreads();
+        } else if (lower == TAIL_LOWER_WAVE) {
+            if (tid < 64) {
+                tail_sync<true>();
+                tail_lower<true, T>(lds, a, inv);
+            }
+            __syncthreads();
+        } else {
+            __syncthreads();
+            tail_lower<false, T>(lds, a, inv);
+        }
+        // level 1 up: correction, black, red
+        if (O.own) {
+            const T* e = tarr(lds, L2, TA_R) + O.e2;
+            const int l2 = L2.cd.ld;
+            T v;
+            if (O.par1 == 0) v = O.pw1[0] * e[0];
+            else if (O.par1 == 1) v = fma(O.pw1[0], e[0], O.pw1[1] * e[1]);
+            else if (O.par1 == 2) v = fma(O.pw1[0], e[0], O.pw1[2] * e[l2]);
+            else v = fma(O.pw1[3], e[l2 + 1], fma(O.pw1[2], e[l2], fma(O.pw1[0], e[0], O.pw1[1] * e[1])));
+            x1 = corrected(x1, v);
+            ya[0] = x1;
+        }
+        __syncthreads();
+        T dne = T(0), dsw = T(0), dnw = T(0), dse = T(0);
+        if (O.own) {
+            dne = ya[ld1 + 1];
+            dsw = ya[-ld1 - 1];
+            dnw = ya[ld1 - 1];
+            dse = ya[1 - ld1];
+            if (!O.red1) {
+                x1 = relaxed(O.r1, b1, full_sum(O.r1, ya[-1], ya[1], ya[-ld1], ya[ld1], dne, dsw, dnw, dse));
+                yb[0] = x1;
+            }
+        }
+        __syncthreads();
+        // a red point's row of yb holds black cells only; its own place there is not read by others yet
+        if (O.red1)
+            yb[0] = relaxed(O.r1, b1, full_sum(O.r1, yb[-1], yb[1], yb[-ld1], yb[ld1], dne, dsw, dnw, dse));
+        __syncthreads();
+    }
+    // level 0 up: correction, black, red
+    if (O.own) {
+        const T e00 = yb[0], e10 = yb[1], e01 = yb[ld1], e11 = yb[ld1 + 1];
+        x[0] = corrected(x[0], O.pw[0] * e00);
+        x[1] = corrected(x[1], O.pw[1] * e00 + O.pw[2] * e10);
+        x[2] = corrected(x[2], O.pw[3] * e00 + O.pw[4] * e01);
+        x[3] = corrected(x[3], O.pw[5] * e00 + O.pw[6] * e10 + O.pw[7] * e01 + O.pw[8] * e11);
+        xa[0] = x[0];
+        xa[1] = x[1];
+        xa[ld] = x[2];
+        xa[ld + 1] = x[3];
+    }
+    __syncthreads();
+    Ring12<T> g{};
+    T r0 = T(0), r3 = T(0);
+    if (O.own) {
+        g = ring(xa, ld);
+        r0 = x[0];
+        r3 = x[3];
+        const T x1n = relaxed(O.r[1], b[1], full_sum(O.r[1], x[0], g.e0, g.s2, x[3], g.e1, g.s1, x[2], g.s3));
+        const T x2n = relaxed(O.r[2], b[2], full_sum(O.r[2], g.w1, x[3], x[0], g.n1, g.n2, g.w0, g.n0, x[1]));
+        x[1] = x1n;
+        x[2] = x2n;
+        xb[1] = x1n;
+        xb[ld] = x2n;
+    }
+    __syncthreads();
+    if (O.own) {
+        x[0] = relaxed(O.r[0], b[0], full_sum(O.r[0], xb[-1], x[1], xb[-ld], x[2], r3, g.s0, g.w1, g.s2));
+        x[3] = relaxed(O.r[3], b[3], full_sum(O.r[3], x[2], xb[ld + 2], x[1], xb[2 * ld + 1], g.n3, r0, g.n1, g.e0));
     }
 }
 
@@ -1063,88 +1350,193 @@ __device__ inline void tail_allreduce(double (&v)[NV], double (*part)[NV]) {
 // bubble against the liquid around it) that one V-cycle resolves poorly;
 // the inner iterations remove them at the cost of a few V-cycles of the
 // smallest levels, all inside one workgroup.
-template <typename T>
-__global__ void __launch_bounds__(TAIL_THREADS) k_tail(TailArgs<T> a, int lds_elems) {
-    if (a.on && !*a.on) return;
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ double inv[COARSEST_MAX * COARSEST_MAX];
+    __shared__ double part_b[TAIL_GROUPS][2];
+    __shared__ double part_a[TAIL_GROUPS][2];
     T* lds = reinterpret_cast<T*>(smem_raw);
     const int tid = threadIdx.x;
-    for (int k = tid; k < lds_elems; k += TAIL_THREADS) lds[k] = T(0);
-    __syncthreads();
-    tail_stage<T>(lds, a);
+    const int live = a.on ? *a.on : 1;
+    // everything the passes read from memory, asked for before the flag is looked at
+    const TailLevel<T>& L0 = a.L[0];
+    const Dims& D0 = L0.d;
+    const int ci = (D0.ni + 1) / 2, cj = (D0.nj + 1) / 2;
+    const int I = tid % ci, J = tid / ci;
+    TailOwn<T> O{};
+    O.own = J < cj;
+    O.p = O.own ? (2 * J + 1) * a.ld0 + 2 * I + 1 : 0;
+    O.p1 = O.own ? (J + 1) * a.ld1 + I + 1 : 0;
+    O.c2 = O.f2 = -1;
+    T b[4] = {T(0), T(0), T(0), T(0)};
+    if (O.own) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 2 * I + (k & 1), j = 2 * J + (k >> 1);
+            O.r[k] = tail_row(L0, i, j);
+            if (i < D0.ni && j < D0.nj) b[k] = L0.b[D0.off(i, j)];
+        }
+        if (a.n > 1) {
+            const Dims& D1 = a.L[1].d;
+            restrict_weights(D1, L0.P, I, J, O.rw);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) O.pw[k] = L0.P.w[k][D1.off(I, J)];
+        }
+        if (a.n > 2) {
+            O.r1 = tail_row(a.L[1], I, J);
+            O.red1 = ((I + J) & 1) == 0;
+            const Dims& D2 = a.L[2].d;
+            T* const* w = a.L[1].P.w;
+            const size_t c = D2.off(I >> 1, J >> 1);
+            const int pi = I & 1, pj = J & 1;
+            O.par1 = pi | pj << 1;
+            O.e2 = toff(a.L[2].cd, I >> 1, J >> 1);
+            O.pw1[0] = w[pi ? (pj ? W_SW : W_XW) : (pj ? W_YS : W_INJ)][c];
+            O.pw1[1] = pi ? w[pj ? W_SE : W_XE][c] : T(0);
+            O.pw1[2] = pj ? w[pi ? W_NW : W_YN][c] : T(0);
+            O.pw1[3] = pi && pj ? w[W_NE][c] : T(0);
+        }
+    }
+    // levels 2.. on one wavefront where they are no larger, level 2 from
+    // registers where the coarsest comes right below it
+    int lower = TAIL_LOWER_ALL;
+    if (a.n > 2) {
+        const Dims& D2 = a.L[2].d;
+        const int n2 = D2.ni * D2.nj;
+        if (n2 <= 64) lower = a.n == 4 ? TAIL_LOWER_OWN : TAIL_LOWER_WAVE;
+        const int I2 = tid % D2.ni, J2 = tid / D2.ni;
+        if (J2 < D2.nj) {
+            restrict_weights(D2, a.L[1].P, I2, J2, O.rw2);
+            O.c2 = toff(a.L[2].cd, I2, J2);
+            O.f2 = (2 * J2 + 1) * a.ld1 + 2 * I2 + 1;
+            O.red2 = ((I2 + J2) & 1) == 0;
+            if (lower == TAIL_LOWER_OWN) O.r2 = tail_row(a.L[2], I2, J2);
+        }
+    }
+    if (!live) return;
+    for (int k = tid; k < lds_elems; k += NT) lds[k] = T(0);
     {
         const Dims& Dc = a.L[a.n - 1].d;
         const int nc = Dc.ni * Dc.nj;
-        double* inv = reinterpret_cast<double*>(lds + a.invbase);
-        for (int k = tid; k < nc * nc; k += TAIL_THREADS) inv[k] = a.inv[k];
+        for (int k = tid; k < nc * nc; k += NT) inv[k] = a.inv[k];
     }
     __syncthreads();
-    const TailLevel<T>& L = a.L[0];
-    const Dims& D = L.cd;
-    const int n = D.ni * D.nj;
-    // level 0's couplings in registers when each thread has at most one cell
-    const bool regs = (D.nj << L.sh) <= TAIL_THREADS;
-    const OwnRow<T> R = regs ? own_row<T>(lds, L) : OwnRow<T>{};
+    // operators and weights of the levels 2..
+    for (int l = 2; l < a.n; ++l) {
+        const TailLevel<T>& L = a.L[l];
+        const int n = L.d.ni * L.d.nj;
+        if (lower != TAIL_LOWER_OWN)
+            for (int k = tid; k < n; k += NT) {
+                const int i = k % L.d.ni, j = k / L.d.ni;
+                const size_t g = L.d.off(i, j), c = L.cd.off(i, j);
+                tarr(lds, L, TA_D)[c] = L.A.diag[g];
+                tarr(lds, L, TA_E)[c] = L.A.cE[g];
+                tarr(lds, L, TA_N)[c] = L.A.cN[g];
+                tarr(lds, L, TA_NE)[c] = L.A.cNE[g];
+                tarr(lds, L, TA_NW)[c] = L.A.cNW[g];
+            }
+        if (l + 1 < a.n) {
+            const TailLevel<T>& Cl = a.L[l + 1];
+            const int nc = Cl.d.ni * Cl.d.nj;
+            for (int k = tid; k < nc; k += NT) {
+                const int ic = k % Cl.d.ni, jc = k / Cl.d.ni;
+                const size_t g = Cl.d.off(ic, jc), c = Cl.cd.off(ic, jc);
+#pragma unroll
+                for (int m = 0; m < 9; ++m) lds[L.wbase + (size_t)m * Cl.cd.alloc_elems() + c] = L.P.w[m][g];
+            }
+        }
+    }
+    __syncthreads();
+    T x[4] = {T(0), T(0), T(0), T(0)};
     if (a.krylov <= 0) {
-        tail_vcycle<T>(lds, a, R, regs);
-        const T* x = tarr(lds, L, TA_R);
-        for (int k = tid; k < n; k += TAIL_THREADS) {
-            const int i = k % D.ni, j = k / D.ni;
-            L.x[L.d.off(i, j)] = x[D.off(i, j)];
+        tail_vcycle(lds, a, O, inv, lower, b, x);
+    } else {
+        // b holds the inner residual; the level's vectors z, q, p and b go to
+        // LDS in linear order for the dots
+        const int n = D0.ni * D0.nj;
+        T *zl = lds + a.lin, *ql = zl + TAIL_MAX, *bl = ql + TAIL_MAX;
+        auto store = [&](T* to, const T (&v)[4]) {
+            if (!O.own) return;
+            const int i = 2 * I, j = 2 * J;
+            T* at = to + j * D0.ni + i;
+            at[0] = v[0];
+            if (i + 1 < D0.ni) at[1] = v[1];
+            if (j + 1 < D0.nj) {
+                at[D0.ni] = v[2];
+                if (i + 1 < D0.ni) at[D0.ni + 1] = v[3];
+            }
+        };
+        T p[4] = {T(0), T(0), T(0), T(0)}, q[4] = {T(0), T(0), T(0), T(0)}, z[4];
+        T* xa = lds + a.x0 + O.p;
+        double pq_prev = 0.0, rr0 = 0.0;
+        for (int it = 0; it < a.krylov; ++it) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) z[k] = T(0);
+            store(bl, b);
+            tail_vcycle(lds, a, O, inv, lower, b, z);
+            store(zl, z);
+            __syncthreads();
+            double v[2];
+            tail_allreduce<NT, 2>(
+                [&](int t, double (&w)[2]) {
+                    const T zp = t < n ? zl[t] : T(0), qv = t < n ? ql[t] : T(0);
+                    const double rp = t < n ? (double)bl[t] : 0.0;
+                    w[0] = (double)zp * (double)qv;
+                    w[1] = rp * rp;
+                },
+                v, part_b);
+            // every thread holds the same sums, so the exits below are uniform:
+            // stop once the inner residual has fallen 1e4 (further iterations
+            // would work on rounding noise, in FP32 above all)
+            if (it == 0) rr0 = v[1];
+            else if (!(v[1] > 1e-8 * rr0)) break;
+            const T beta = (it > 0 && pq_prev > 0.0) ? (T)(-v[0] / pq_prev) : T(0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p[k] = z[k] + beta * p[k];
+            if (O.own) {
+                xa[0] = p[0];
+                xa[1] = p[1];
+                xa[a.ld0] = p[2];
+                xa[a.ld0 + 1] = p[3];
+            }
+            store(zl, p);
+            __syncthreads();
+            if (O.own) {
+                T s[4];
+                block_sums(O, ring(xa, a.ld0), p, s);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) q[k] = O.r[k].d * p[k] - s[k];
+            }
+            store(ql, q);
+            __syncthreads();
+            double v2[2];
+            tail_allreduce<NT, 2>(
+                [&](int t, double (&w)[2]) {
+                    const T pp = t < n ? zl[t] : T(0), qv = t < n ? ql[t] : T(0);
+                    const double rp = t < n ? (double)bl[t] : 0.0;
+                    w[0] = (double)pp * rp;
+                    w[1] = (double)pp * (double)qv;
+                },
+                v2, part_a);
+            const double al = v2[0] / v2[1];
+            if (!(v2[1] > 0.0) || !(fabs(al) < 1e30)) break;
+            const T alpha = (T)al;
+            pq_prev = v2[1];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                x[k] += alpha * p[k];
+                b[k] -= alpha * q[k];
+            }
         }
-        return;
     }
-    // inner flexible CG; level lt has at most TAIL_THREADS points, one per thread
-    __shared__ double part_b[TAIL_THREADS / 64][2];
-    __shared__ double part_a[TAIL_THREADS / 64][2];
-    const size_t ld = D.ld;
-    const bool own = tid < n;
-    const size_t p = own ? D.off(tid % D.ni, tid / D.ni) : 0;
-    T* res = tarr(lds, L, TA_B);  // the V-cycle's right-hand side
-    const T* z = tarr(lds, L, TA_R);
-    T* pv = lds + a.pbase;
-    const T* d = tarr(lds, L, TA_D);
-    const T* e = tarr(lds, L, TA_E);
-    const T* nn = tarr(lds, L, TA_N);
-    const T* ne = tarr(lds, L, TA_NE);
-    const T* nw = tarr(lds, L, TA_NW);
-    T xacc = T(0), qv = T(0);
-    double pq_prev = 0.0, rr0 = 0.0;
-    for (int it = 0; it < a.krylov; ++it) {
-        tail_vcycle<T>(lds, a, R, regs);  // ends with a barrier
-        const T zp = own ? z[p] : T(0);
-        const double rp = own ? (double)res[p] : 0.0;
-        double v[2] = {(double)zp * (double)qv, rp * rp};
-        tail_allreduce<2>(v, part_b);
-        // every thread holds the same sums, so the exits below are uniform:
-        // stop once the inner residual has fallen 1e4 (further iterations
-        // would work on rounding noise, in FP32 above all)
-        if (it == 0) rr0 = v[1];
-        else if (!(v[1] > 1e-8 * rr0)) break;
-        const T beta = (it > 0 && pq_prev > 0.0) ? (T)(-v[0] / pq_prev) : T(0);
-        if (own) pv[p] = zp + beta * pv[p];
-        __syncthreads();
-        T pp = T(0);
-        if (own) {
-            pp = pv[p];
-            const T s = e[p - 1] * pv[p - 1] + e[p] * pv[p + 1] + nn[p - ld] * pv[p - ld] + nn[p] * pv[p + ld] +
-                        ne[p] * pv[p + ld + 1] + ne[p - ld - 1] * pv[p - ld - 1] + nw[p] * pv[p + ld - 1] +
-                        nw[p - ld + 1] * pv[p - ld + 1];
-            qv = d[p] * pp - s;
+    if (O.own) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int i = 2 * I + (k & 1), j = 2 * J + (k >> 1);
+            if (i < D0.ni && j < D0.nj) L0.x[D0.off(i, j)] = x[k];
         }
-        double v2[2] = {(double)pp * rp, (double)pp * (double)qv};
-        tail_allreduce<2>(v2, part_a);
-        const double al = v2[0] / v2[1];
-        if (!(v2[1] > 0.0) || !(fabs(al) < 1e30)) break;
-        const T alpha = (T)al;
-        pq_prev = v2[1];
-        if (own) {
-            xacc += alpha * pp;
-            res[p] -= alpha * qv;
-        }
-        __syncthreads();
     }
-    if (own) L.x[L.d.off(tid % D.ni, tid / D.ni)] = xacc;
 }
 
 // coarsest-only hierarchy (grids of at most COARSEST_MAX cells): the dense
@@ -1188,6 +1580,64 @@ inline Dims compact(const Dims& d) {
     return c;
 }
 
+// The tail's levels and their LDS: level 0 two arrays with a ring of zeros,
+// level 1 two, the levels below it their operators, vectors and weights.  A
+// tail is refused by the size of all its levels' operators, vectors and
+// weights, whatever of that sits in registers.
+template <typename T>
+int tail_layout(Ctx* c, int lt, const int* on, TailArgs<T>& ta, size_t& lds) {
+    const int nl = c->nlev;
+    ta.n = nl - lt;
+    if (ta.n > MAX_TAIL) {
+        set_error("multigrid: too many tail levels");
+        return SG_ERR_STATE;
+    }
+    ta.krylov = c->prm.mg_coarse_krylov;
+    ta.inv = c->coarse_inv;
+    ta.on = on;
+    const Dims &d0 = c->lev[lt].d;
+    const int ci = (d0.ni + 1) / 2, cj = (d0.nj + 1) / 2;
+    int off = 0;
+    auto take = [&](int n) {
+        const int at = off;
+        off += n;
+        return at;
+    };
+    ta.ld0 = 2 * ci + 2;
+    ta.x0 = take(ta.ld0 * (2 * cj + 2));
+    ta.x1 = take(ta.ld0 * (2 * cj + 2));
+    ta.ld1 = ci + 2;
+    ta.y0 = take(ta.ld1 * (cj + 2));
+    ta.y1 = take(ta.ld1 * (cj + 2));
+    ta.lin = take(ta.krylov > 0 ? 3 * TAIL_MAX : 0);
+    size_t all = ta.krylov > 0 ? compact(d0).alloc_elems() : 0;
+    for (int k = 0; k < ta.n; ++k) {
+        const Level& L = c->lev[lt + k];
+        TailLevel<T>& t = ta.L[k];
+        t.d = L.d;
+        t.cd = compact(L.d);
+        t.sh = 0;
+        while ((1 << t.sh) < L.d.ni) ++t.sh;
+        t.A = opv(Acc<T>::op(L));
+        t.P = Acc<T>::pr(L);
+        t.x = Acc<T>::vec(L).x;
+        t.b = Acc<T>::vec(L).b;
+        const int next = k + 1 < ta.n ? 9 * (int)compact(c->lev[lt + k + 1].d).alloc_elems() : 0;
+        if (k >= 2) {
+            t.base = take(TA_COUNT * (int)t.cd.alloc_elems());
+            t.wbase = take(next);
+        }
+        all += 8 * t.cd.alloc_elems() + next;
+    }
+    const size_t nc = (size_t)c->lev[nl - 1].d.ni * c->lev[nl - 1].d.nj;
+    if (all * sizeof(T) + nc * nc * sizeof(double) > TAIL_LDS_MAX) {
+        set_error("multigrid: tail levels exceed the LDS budget");
+        return SG_ERR_STATE;
+    }
+    lds = (size_t)off;
+    return SG_OK;
+}
+
 // z = M^{-1} r ; fine-level dots (r,z), (z,q) go to the partials slot S;
 // V = type of the PCG vectors r, z, q; every kernel returns at once while
 // *on == 0 (a converged PCG)
@@ -1223,52 +1673,19 @@ int vcycle(Ctx* c, const V* r, V* z, const V* q, Slots S, int* dots_done, const 
     }
     // tail
     TailArgs<T> ta{};
-    ta.n = nl - lt;
-    if (ta.n > MAX_TAIL) {
-        set_error("multigrid: too many tail levels");
-        return SG_ERR_STATE;
+    size_t tail_lds = 0;
+    int rc = tail_layout<T>(c, lt, on, ta, tail_lds);
+    if (rc) return rc;
+    {
+        const Dims& d = c->lev[lt].d;
+        const int blocks = ((d.ni + 1) / 2) * ((d.nj + 1) / 2);
+        if (blocks <= TAIL_NT)
+            hipLaunchKernelGGL((k_tail<T, TAIL_NT>), dim3(1), dim3(TAIL_NT), tail_lds * sizeof(T), s, ta,
+                               (int)tail_lds);
+        else
+            hipLaunchKernelGGL((k_tail<T, TAIL_NT_MAX>), dim3(1), dim3(TAIL_NT_MAX), tail_lds * sizeof(T), s, ta,
+                               (int)tail_lds);
     }
-    int off = 0;
-    for (int k = 0; k < ta.n; ++k) {
-        const Level& L = c->lev[lt + k];
-        TailLevel<T>& t = ta.L[k];
-        t.d = L.d;
-        t.cd = compact(L.d);
-        t.sh = 0;
-        while ((1 << t.sh) < L.d.ni) ++t.sh;
-        t.base = off;
-        off += TA_COUNT * (int)t.cd.alloc_elems();
-        t.A = opv(Acc<T>::op(L));
-        t.P = Acc<T>::pr(L);
-        t.x = Acc<T>::vec(L).x;
-        t.b = Acc<T>::vec(L).b;
-        if (k + 1 < ta.n) {
-            t.wbase = off;
-            off += 9 * (int)compact(c->lev[lt + k + 1].d).alloc_elems();
-        }
-    }
-    ta.krylov = c->prm.mg_coarse_krylov;
-    ta.pbase = off;
-    if (ta.krylov > 0) {
-        if (c->lev[lt].d.ni * c->lev[lt].d.nj > TAIL_THREADS) {
-            set_error("multigrid: the first tail level exceeds one point per thread");
-            return SG_ERR_STATE;
-        }
-        off += (int)compact(c->lev[lt].d).alloc_elems();
-    }
-    // the FP64 inverse: 8-byte aligned, sizeof(double) / sizeof(T) slots per entry
-    constexpr int per = (int)(sizeof(double) / sizeof(T));
-    off = (off + per - 1) / per * per;
-    ta.invbase = off;
-    off += per * (int)(c->lev[nl - 1].d.ni * c->lev[nl - 1].d.nj) * (int)(c->lev[nl - 1].d.ni * c->lev[nl - 1].d.nj);
-    const size_t lds_bytes = (size_t)off * sizeof(T);
-    if (lds_bytes > TAIL_LDS_MAX) {
-        set_error("multigrid: tail levels exceed the LDS budget");
-        return SG_ERR_STATE;
-    }
-    ta.inv = c->coarse_inv;
-    ta.on = on;
-    hipLaunchKernelGGL((k_tail<T>), dim3(1), dim3(TAIL_THREADS), lds_bytes, s, ta, off);
     // up: level l reads x_l from the down pass and e_{l+1}; writes its own
     // correction into r_l (its solution for the level above)
     for (int l = lt - 1; l >= 0; --l) {
