@@ -765,14 +765,7 @@ int sg_clsvof_advect_resident(sg_ctx* ctx, double dt, double time, const sg_clsv
         set_error("sg_clsvof_advect: dt must be >= 0");
         return SG_ERR_ARG;
     }
-    // Depthw + etau of each sub-step (X_Sweep, Clsvof_Mod.f90:1057-1059)
-    std::vector<double> levels(p->nsub);
-    const double dtv = dt / (double)p->nsub;
-    for (int k = 1; k <= p->nsub; ++k) {
-        const double etau = p->amp * std::sin(p->kw * c->cls.xw - p->omega * (time + (double)k * dtv));
-        levels[k - 1] = p->depth + etau;
-    }
-    int rc = clsvof_advect(c, dt, p->nsub, levels.data());
+    int rc = clsvof_advect(c, dt, p->nsub);
     if (rc) return rc;
     SG_HIP(hipGetLastError());
     c->built = 0;

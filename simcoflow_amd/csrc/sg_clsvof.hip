@@ -3,18 +3,17 @@
 // One call advances vof and phi over dt in nsub sub-steps (Coupled_LS_VOF,
 // Clsvof_Mod.f90:730-959).  Each sub-step runs these launches:
 //
-//   k_recon      PLIC reconstruction (Interface_Reconstruct :1250-1321):
-//                classify the cells and list the interface ones,
-//   k_recon_ifc  then their normals and plane constants, packed one per lane
-//   k_dis_fix    cells whose plane constant the reference leaves stale
-//   k_flux_pre   PLIC face fluxes of the listed cells, packed one per lane
-//   k_sweep      first sweep, implicit divergence (:798-823 / :862-888)
-//   k_bc         boundary copy (Boundary_Condition :961-973)
-//   k_recon, k_recon_ifc, k_dis_fix, k_flux_pre
+//   k_recon      PLIC reconstruction (Interface_Reconstruct :1250-1321): find
+//                the interface cells, then, packed one per lane, their normals,
+//                plane constants and the PLIC face fluxes of the coming sweep
+//                (k_recon_ifc: on the cells the last scan listed)
+//   k_sweep      first sweep, implicit divergence (:798-823 / :862-888), with
+//                the boundary copy (Boundary_Condition :961-973)
+//   k_recon
 //   k_sweep      second sweep, explicit divergence (:834-858 / :898-929)
-//   k_bc, k_recon (+ interface bit mask and source list), k_recon_ifc, k_dis_fix
-//   k_rd_scatter, k_rd_dilate, k_redistance_far, k_redistance_band: level
-//                set from the PLIC segments (Redistance :1525-1708)
+//   k_recon (+ interface bit mask and source list)
+//   k_rd_scatter, k_redistance: level set from the PLIC segments (Redistance
+//                :1525-1708)
 //
 // The reference's sweeps walk each row in order and update cells in place;
 // every face flux they use depends only on data from before the sweep, so a
@@ -29,6 +28,8 @@
 //
 // This file is compiled with FP contraction off: every sum and product
 // rounds as the reference writes it.
+#include <type_traits>
+
 #include "sg_internal.hpp"
 #include "sg_poly.hpp"
 
@@ -571,181 +572,24 @@ __device__ __forceinline__ void plane_pick(double vf, double vs, double hy, doub
     }
 }
 
-// wavefront-aggregated append of `value` to list where pred holds (one
-// atomic per wavefront); every lane of the wavefront must call it
-__device__ __forceinline__ void append(bool pred, unsigned* count, int* list, int value) {
-    const unsigned long long b = __ballot(pred);
-    if (!b) return;
-    const int lane = __lane_id();
-    const int leader = __ffsll((long long)b) - 1;
-    unsigned base = 0;
-    if (lane == leader) base = atomicAdd(count, (unsigned)__popcll(b));
-    base = __shfl(base, leader);
-    if (pred) list[base + (unsigned)__popcll(b & ((1ull << lane) - 1ull))] = value;
+// One bit per cell (a 64-bit word per 64 cells of a row) for what later kernels
+// ask of every cell, written by whoever has the cell's vof in a register (a
+// sweep, or a scanning reconstruction) so that nobody reads vof and vofS again
+// only to find the interface.
+enum { BIT_LIST = 0, BIT_SRC, BIT_GAS, BIT_LIQ, NBITS };
+struct Bits {
+    unsigned long long* w[NBITS];
+    int mw;  // words per row
+};
+// BIT_LIST: an interface cell, or one whose face fluxes need the PLIC geometry
+// (vof_flux's branch); BIT_SRC: a source of re-distancing; BIT_GAS, BIT_LIQ:
+// empty or full cells, which take the band value away from the interface
+__device__ __forceinline__ bool bit_list(double f, double vs) {
+    return recon_class(f, vs) != 0 || !(f >= (1.0 - VOFEPS) || f <= VOFEPS);
 }
-
-// Interface_Reconstruct.  Interface cells get their normal and plane
-// constant; three-phase cells whose Ridders search leaves the plane constant
-// unassigned (the reference then keeps the previous cell's) are flagged in
-// `stale` and listed for k_dis_fix.  full_out: also write n = (0,1) for the
-// other cells (the PCell%nx/ny output).  With mask != null the kernel also
-// writes the re-distancing source mask (vofeps < vof < 1-vofeps-vofS, one bit
-// per cell, one 64-bit word per wavefront and row) and lists those cells.
-// cnt[0]: sources listed, cnt[1]: stale cells listed, cnt[2]: interface
-// cells listed.
-//
-// This scan is bound by its appends, not its bytes: every workgroup that
-// lists a cell takes one atomic on a counter all workgroups share.  So a
-// workgroup covers 64 x 64 cells, each thread RECON_R rows, and lists all of
-// them with one scan and one atomic per list (the two per-thread counts
-// packed in one word, low and high 16 bits: at most 4096 of each per
-// workgroup).
-constexpr int RECON_TY = 16;  // wavefronts per k_recon workgroup
-constexpr int RECON_R = 4;    // rows per thread: a workgroup covers 64 x (RECON_TY * RECON_R) cells
-__global__ void __launch_bounds__(64 * RECON_TY) k_recon(ClsGeo G, const double* __restrict__ vof, Planes P,
-                                                         int full_out,
-                                               unsigned long long* __restrict__ mask, int mw,
-                                               int* __restrict__ srcs, int* __restrict__ ifc,
-                                               unsigned* __restrict__ cnt) {
-    __shared__ unsigned wsum[RECON_TY], wbase_i[RECON_TY], wbase_s[RECON_TY], gbase[2];
-    const int lane = threadIdx.x, w = threadIdx.y;
-    const int i = blockIdx.x * 64 + lane + 1;
-    const int j0 = blockIdx.y * (RECON_TY * RECON_R) + w + 1;
-    // every row's operands loaded before any test
-    double vf[RECON_R], vs[RECON_R];
-#pragma unroll
-    for (int r = 0; r < RECON_R; ++r) {
-        const int j = j0 + r * RECON_TY;
-        const bool in = i <= G.ni && j <= G.nj;
-        const size_t c = in ? cix(G, i, j) : 0;
-        vf[r] = in ? vof[c] : 0.0;
-        vs[r] = in ? G.vofS[c] : 0.0;
-    }
-    unsigned list_i = 0, list_s = 0;  // bit r: row r's cell goes to ifc / srcs
-#pragma unroll
-    for (int r = 0; r < RECON_R; ++r) {
-        const int j = j0 + r * RECON_TY;
-        const bool in = i <= G.ni && j <= G.nj;
-        const bool src = in && (0.0 + VOFEPS) < vf[r] && vf[r] < (1.0 - VOFEPS - vs[r]);
-        const bool itf = in && recon_class(vf[r], vs[r]) != 0;
-        const bool heavy = in && !(vf[r] >= (1.0 - VOFEPS) || vf[r] <= VOFEPS);  // vof_flux's PLIC branch
-        if (in && !itf && full_out) {
-            const size_t c = cix(G, i, j);
-            P.nx[c] = 0.0;
-            P.ny[c] = 1.0;
-        }
-        if (itf || heavy) list_i |= 1u << r;
-        if (mask) {
-            // one wavefront covers 64 consecutive i of row j
-            const unsigned long long bits = __ballot(src);
-            if (lane == 0 && j <= G.nj) mask[(size_t)(j - 1) * mw + blockIdx.x] = bits;
-            if (src) list_s |= 1u << r;
-        }
-    }
-    // exclusive offsets of this thread's entries in the workgroup's share of
-    // each list: an inclusive scan of the packed counts over the wavefront,
-    // then over the wavefronts
-    const unsigned own = (unsigned)__popc(list_i) | ((unsigned)__popc(list_s) << 16);
-    unsigned incl = own;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned t = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += t;
-    }
-    if (lane == 63) wsum[w] = incl;
-    __syncthreads();
-    if (w == 0 && lane == 0) {
-        unsigned si = 0, ss = 0;
-        for (int k = 0; k < RECON_TY; ++k) {
-            wbase_i[k] = si;
-            wbase_s[k] = ss;
-            si += wsum[k] & 0xFFFFu;
-            ss += wsum[k] >> 16;
-        }
-        gbase[0] = si ? atomicAdd(cnt + 2, si) : 0u;
-        gbase[1] = ss ? atomicAdd(cnt, ss) : 0u;
-    }
-    __syncthreads();
-    const unsigned excl = incl - own;
-    unsigned oi = gbase[0] + wbase_i[w] + (excl & 0xFFFFu);
-    unsigned os = gbase[1] + wbase_s[w] + (excl >> 16);
-#pragma unroll
-    for (int r = 0; r < RECON_R; ++r) {
-        const int c = (int)cix(G, i, j0 + r * RECON_TY);
-        if (list_i >> r & 1u) ifc[oi++] = c;
-        if (list_s >> r & 1u) srcs[os++] = c;
-    }
-}
-
-// The interface cells listed by k_recon, packed one per lane: the normal and
-// plane constant cost the same per cell wherever a cell lies, and packing
-// keeps the wavefronts of bulk liquid and gas out of that work.
-__global__ void __launch_bounds__(256) k_recon_ifc(ClsGeo G, const double* __restrict__ vof,
-                                                   const double* __restrict__ phi, Planes P,
-                                                   unsigned char* __restrict__ stale, const int* __restrict__ ifc,
-                                                   const unsigned* __restrict__ nifc, int* __restrict__ stales,
-                                                   unsigned* __restrict__ cnt) {
-    const unsigned n = *nifc;
-    for (unsigned base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
-        const unsigned t = base + threadIdx.x;
-        bool st = false;
-        int c = 0;
-        if (t < n) c = ifc[t];
-        const double vf = t < n ? vof[c] : 0.0, vs = t < n ? G.vofS[c] : 0.0;
-        const int cl = t < n ? recon_class(vf, vs) : 0;
-        if (cl) {
-            const int i = c % G.ni + 1, j = c / G.ni + 1;
-            double nx, ny, d = 0.0;
-            if (i > 1 && i < G.ni && j > 1 && j < G.nj)
-                final_interior(G, vof, phi, i, j, nx, ny);
-            else if (i == 1 || i == G.ni)
-                final_side(G, vof, phi, i, j, nx, ny);
-            else
-                final_topbottom(G, vof, phi, i, j, nx, ny);
-            const double hx = G.dx[i - 1], hy = G.dy[j - 1];
-            if (cl == 1)
-                d = plic_distance(vf, nx, ny, hx, hy);
-            else
-                st = !distance_fluid(G.nxS[c], G.nyS[c], G.phiS[c], nx, ny, vf, hx, hy, d);
-            P.nx[c] = nx;
-            P.ny[c] = ny;
-            P.dis[c] = d;
-            if (cl == 2) stale[c] = st ? 1 : 0;
-        }
-        append(st, cnt + 1, stales, c);
-    }
-}
-
-// Cells whose plane constant the reference leaves stale take the value of
-// the nearest earlier cell in its loop order (i outer, j inner) that has one.
-__global__ void __launch_bounds__(256) k_dis_fix(ClsGeo G, const double* __restrict__ vof,
-                                                 const unsigned char* __restrict__ stale,
-                                                 const int* __restrict__ list, const unsigned* __restrict__ cnt,
-                                                 double* __restrict__ dis) {
-    const unsigned n = cnt[1];
-    for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        const int c0 = list[t];
-        int pi = c0 % G.ni + 1, pj = c0 / G.ni + 1;
-        double d = 0.0;
-        for (;;) {
-            if (pj > 1) {
-                --pj;
-            } else if (pi > 1) {
-                --pi;
-                pj = G.nj;
-            } else {
-                break;  // before the first cell: the reference's uninitialised local
-            }
-            const size_t p = cix(G, pi, pj);
-            const double vf = vof[p], vs = G.vofS[p];
-            const int cl = recon_class(vf, vs);
-            if (cl == 2 && stale[p]) continue;
-            d = cl ? dis[p] : default_dis(vf, vs, G.dy[pj - 1]);
-            break;
-        }
-        dis[c0] = d;
-    }
-}
+__device__ __forceinline__ bool bit_src(double f, double vs) { return (0.0 + VOFEPS) < f && f < (1.0 - VOFEPS - vs); }
+__device__ __forceinline__ bool bit_gas(double f) { return f <= VOFEPS; }
+__device__ __forceinline__ bool bit_liq(double f, double vs) { return f >= (1.0 - VOFEPS - vs); }
 
 // Boundary_Condition (:961-973) on two arrays: every ring cell takes its
 // value from an interior cell, so the copy is race-free in place.
@@ -792,6 +636,8 @@ struct Line {
         const bool on = G.vflag[cix(G, b, af)];
         return a == 0 || on ? w : 0.0;
     }
+    // the same through a face that is not masked
+    __device__ double raw(int a) const { return X ? G.u[gix(G, a, b)] : G.v[gix(G, b, a)]; }
     __device__ double ap(int a) const { return X ? G.aE[gix(G, a, b)] : G.aN[gix(G, b, a)]; }
     __device__ double am(int a) const { return X ? G.aW[gix(G, a, b)] : G.aS[gix(G, b, a)]; }
     __device__ double h(int a) const { return X ? G.dx[a - 1] : G.dy[a - 1]; }
@@ -830,31 +676,11 @@ __device__ double plic_face_flux(int side, double nxx, double nyy, double diss, 
 struct SweepIn {
     const double* vof;
     const double* phi;
-    Planes pl;
-    // PLIC fluxes precomputed by k_flux_pre: the sweep itself holds none of
-    // the plane geometry, which keeps it free of scratch and light on registers
+    // PLIC fluxes prepared by the reconstruction: the sweep itself holds none
+    // of the plane geometry, which keeps it free of scratch and light on registers
     const double* fr;
     const double* fl;
 };
-
-// the PLIC flux of vof_flux through face a with upwind cell a (far face of
-// cell a) and through face a with upwind cell a+1 (near face of cell a+1)
-template <bool X>
-__device__ double plic_far(const Line<X>& L, const SweepIn& s, int a, size_t c, double f, double w, double dtv) {
-    const ClsGeo& G = L.G;
-    const double hx = X ? G.dx[a - 1] : G.dx[L.b - 1], hy = X ? G.dy[L.b - 1] : G.dy[a - 1];
-    double nx, ny, d;
-    plane_of(G, s.pl, c, f, hy, nx, ny, d);
-    return plic_face_flux<X>(1, nx, ny, d, f, G.nxS[c], G.nyS[c], G.phiS[c], G.vofS[c], hx, hy, w * dtv);
-}
-template <bool X>
-__device__ double plic_near(const Line<X>& L, const SweepIn& s, int a, size_t c, double f, double w, double dtv) {
-    const ClsGeo& G = L.G;
-    const double hx = X ? G.dx[a] : G.dx[L.b - 1], hy = X ? G.dy[L.b - 1] : G.dy[a];
-    double nx, ny, d;
-    plane_of(G, s.pl, c, f, hy, nx, ny, d);
-    return -plic_face_flux<X>(-1, nx, ny, d, f, G.nxS[c], G.nyS[c], G.phiS[c], G.vofS[c], hx, hy, -w * dtv);
-}
 
 // vof_flux (X_Sweep :1014-1051) once the upwind cell of the face is known:
 // f, vsU its vof and vofS, apU its aperture of the face, plic the PLIC flux
@@ -901,140 +727,384 @@ __device__ double ls_flux_first(const Line<X>& L, const double* phi, double dtv)
     return l * w * dtv;
 }
 
-// level-set flux through the last face (:1111-1123 / :1231-1243)
-template <bool X>
-__device__ double ls_flux_last(const Line<X>& L, const double* phi, double dtv) {
-    const int n = L.na();
-    const double w = L.vel(n);
-    const double pn = phi[L.c(n)], pm = phi[L.c(n - 1)];
-    double l;
-    if (w > 0.0)
-        l = pn + L.h(n) / 2.0 * (1.0 - w * dtv / L.h(n)) * (pn - pm) / (L.pos(n) - L.pos(n - 1));
-    else
-        l = pn - L.h(n - 1) / 2.0 * (1.0 + w * dtv / L.h(n - 1)) * (pn - pm) / (L.pos(n) - L.pos(n - 1));
-    return l * w * dtv;
+__device__ __forceinline__ unsigned long long lane_word(unsigned long long v, int lane) {
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)v, lane);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(v >> 32), lane);
+    return (unsigned long long)hi << 32 | lo;
 }
 
-// The PLIC face fluxes of a sweep for the listed cells (VOFEPS < vof <
-// 1-VOFEPS), packed one per lane: the far-face flux where the cell is upwind
-// of its far face, the near-face flux where it is upwind of its near face --
-// exactly the values vof_flux would compute for them in the sweep.
+// ---- reconstruction ---------------------------------------------------------
+
+// the sweep whose PLIC face fluxes a reconstruction prepares
+enum FluxDir { FLUX_NONE = 0, FLUX_X, FLUX_Y };
+
+struct ReconOut {
+    Planes P;
+    double* fr;
+    double* fl;
+};
+
+// the PLIC face fluxes of cell c (VOFEPS < vof < 1-VOFEPS) with its plane: the
+// far-face flux where the cell is upwind of its far face, the near-face flux
+// where it is upwind of its near face -- exactly the values vof_flux would
+// compute for them in the sweep
 template <bool X>
-__global__ void __launch_bounds__(256) k_flux_pre(ClsGeo G, SweepIn s, double dtv, const int* __restrict__ list,
-                                                  const unsigned* __restrict__ cnt, double* __restrict__ fr,
-                                                  double* __restrict__ fl) {
-    const unsigned n = cnt[2];
-    for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
-        const int c = list[t];
-        const double f = s.vof[c];
-        if (f >= (1.0 - VOFEPS) || f <= VOFEPS) continue;  // not vof_flux's PLIC branch
-        const int i = c % G.ni + 1, j = c / G.ni + 1;
-        const Line<X> L{G, X ? j : i};
-        const int a = X ? i : j;
-        const double w = L.vel(a);
-        if (X ? (w >= 0.0) : (w > 0.0)) fr[c] = plic_far<X>(L, s, a, c, f, w, dtv);
-        const double w0 = L.vel(a - 1);
-        if (!(X ? (w0 >= 0.0) : (w0 > 0.0))) fl[c] = plic_near<X>(L, s, a - 1, c, f, w0, dtv);
+__device__ __forceinline__ void cell_fluxes(const ClsGeo& G, int c, double f, double nx, double ny, double d,
+                                            double dtv, double* __restrict__ fr, double* __restrict__ fl) {
+    if (f >= (1.0 - VOFEPS) || f <= VOFEPS) return;  // not vof_flux's PLIC branch
+    const int i = c % G.ni + 1, j = c / G.ni + 1;
+    const Line<X> L{G, X ? j : i};
+    const int a = X ? i : j;
+    const double hx = G.dx[i - 1], hy = G.dy[j - 1];
+    const double nxs = G.nxS[c], nys = G.nyS[c], phis = G.phiS[c], vs = G.vofS[c];
+    const double w = L.vel(a), w0 = L.vel(a - 1);
+    if (X ? (w >= 0.0) : (w > 0.0))
+        fr[c] = plic_face_flux<X>(1, nx, ny, d, f, nxs, nys, phis, vs, hx, hy, w * dtv);
+    if (!(X ? (w0 >= 0.0) : (w0 > 0.0)))
+        fl[c] = -plic_face_flux<X>(-1, nx, ny, d, f, nxs, nys, phis, vs, hx, hy, -w0 * dtv);
+}
+
+// Interface_Reconstruct of cell c: its normal and plane constant where it is an
+// interface cell, then its fluxes.  A three-phase cell whose Ridders search
+// leaves the plane constant unassigned takes the one of the nearest earlier
+// cell in the reference's loop order (i outer, j inner) that assigns it (the
+// reference keeps the previous cell's): the walk back works those cells out
+// again from the same fields, which costs the few lanes that need it a cell's
+// chain more and every other reconstruction nothing.  (As a kernel over a list
+// of such cells it took 3.6 us of each reconstruction at 333 x 171, empty or not.)
+template <int DIR>
+__device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __restrict__ vof,
+                                           const double* __restrict__ phi, const ReconOut& O, double dtv, int c,
+                                           bool full) {
+    const double vf = vof[c];
+    double nx = 0.0, ny = 1.0, d = 0.0;
+    int i = c % G.ni + 1, j = c / G.ni + 1;
+    bool own = true, itf = false;
+    for (;;) {
+        const size_t p = cix(G, i, j);
+        const double v = vof[p], vs = G.vofS[p];
+        const int cl = recon_class(v, vs);
+        const double hx = G.dx[i - 1], hy = G.dy[j - 1];
+        bool set = true;
+        if (cl) {
+            double mx, my;
+            if (i > 1 && i < G.ni && j > 1 && j < G.nj)
+                final_interior(G, vof, phi, i, j, mx, my);
+            else if (i == 1 || i == G.ni)
+                final_side(G, vof, phi, i, j, mx, my);
+            else
+                final_topbottom(G, vof, phi, i, j, mx, my);
+            if (cl == 1)
+                d = plic_distance(v, mx, my, hx, hy);
+            else
+                set = distance_fluid(G.nxS[p], G.nyS[p], G.phiS[p], mx, my, v, hx, hy, d);
+            if (own) {
+                nx = mx;
+                ny = my;
+                itf = true;
+            }
+        } else {
+            d = default_dis(v, vs, hy);
+        }
+        if (set) break;
+        own = false;
+        if (j > 1) {
+            --j;
+        } else if (i > 1) {
+            --i;
+            j = G.nj;
+        } else {
+            d = 0.0;  // before the first cell: the reference's uninitialised local
+            break;
+        }
+    }
+    if (itf || full) {
+        O.P.nx[c] = nx;
+        O.P.ny[c] = ny;
+    }
+    if (itf) O.P.dis[c] = d;
+    if (DIR != FLUX_NONE) cell_fluxes<DIR == FLUX_X>(G, c, vf, nx, ny, d, dtv, O.fr, O.fl);
+}
+
+// Interface_Reconstruct over the grid: a workgroup lists the cells of its 64 x
+// 64 that BIT_LIST names in LDS and works on them packed one per lane -- the
+// geometry costs the same per cell wherever a cell lies, and packing keeps the
+// wavefronts of bulk liquid and gas out of it.  SCAN: the bits are not there
+// yet (a call's first reconstruction, or vofS has moved since the sweep), so
+// they come from vof and vofS here and are written for the kernels after.
+// full: also n = (0,1) for the other cells (the PCell%nx/ny output).  With
+// srcs the sources of re-distancing are appended to it, one atomic a workgroup.
+//
+// Bound by the latency of one cell's chain of divisions and square roots, with
+// SCAN also by 16 bytes a cell.  As a scan, a kernel over the listed cells, one
+// over those with a stale plane constant and one for the fluxes it took 19.6 us
+// at 333 x 171 and 37.3 us at 2048^2; in one, scanning, 16.6 and 34 us; with the
+// bits of the sweep before it 10.9 and 13.9 us (17.1 us listing the sources).
+constexpr int RECON_NT = 256;
+constexpr int RECON_H = 64;  // rows per workgroup: one a lane when the words are listed
+template <int DIR, bool SCAN>
+__global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __restrict__ vof,
+                                                    const double* __restrict__ phi, ReconOut O, Bits B, double dtv,
+                                                    int full, int* __restrict__ srcs, unsigned* __restrict__ nsrc) {
+    constexpr int NW = RECON_NT / 64, R = RECON_H / NW;
+    __shared__ unsigned long long words[2][SCAN ? RECON_H : 1];
+    __shared__ unsigned short list[64 * RECON_H];
+    __shared__ unsigned gbase;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i0 = blockIdx.x * 64, jb = blockIdx.y * RECON_H;
+    if (SCAN) {
+        const int i = i0 + lane + 1;
+        // every row's operands loaded before any test
+        double vf[R], vs[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int j = jb + r * NW + w + 1;
+            const bool in = i <= G.ni && j <= G.nj;
+            const size_t c = in ? cix(G, i, j) : 0;
+            vf[r] = in ? vof[c] : 0.0;
+            vs[r] = in ? G.vofS[c] : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int row = r * NW + w, j = jb + row + 1;
+            const bool in = i <= G.ni && j <= G.nj;
+            unsigned long long b[NBITS];
+            b[BIT_LIST] = __ballot(in && bit_list(vf[r], vs[r]));
+            b[BIT_SRC] = __ballot(in && bit_src(vf[r], vs[r]));
+            b[BIT_GAS] = __ballot(in && bit_gas(vf[r]));
+            b[BIT_LIQ] = __ballot(in && bit_liq(vf[r], vs[r]));
+            if (lane == 0) {
+                words[0][row] = b[BIT_LIST];
+                words[1][row] = b[BIT_SRC];
+            }
+            if (lane < NBITS && j <= G.nj) {
+                const unsigned long long v = lane == 0 ? b[0] : lane == 1 ? b[1] : lane == 2 ? b[2] : b[3];
+                B.w[lane][(size_t)(j - 1) * B.mw + blockIdx.x] = v;
+            }
+        }
+        __syncthreads();
+    }
+    // one row's word a lane, in every wavefront
+    const bool row_in = jb + lane < G.nj;
+    unsigned long long wl = 0ull, ws = 0ull;
+    if (SCAN) {
+        wl = words[0][lane];
+        if (srcs) ws = words[1][lane];
+    } else if (row_in) {
+        const size_t at = (size_t)(jb + lane) * B.mw + blockIdx.x;
+        wl = B.w[BIT_LIST][at];
+        if (srcs) ws = B.w[BIT_SRC][at];
+    }
+    // where each row's cells start in the two lists: an inclusive scan of the
+    // packed counts (low and high 16 bits, at most 4096 of each) over the rows
+    const unsigned own = (unsigned)__popcll(wl) | ((unsigned)__popcll(ws) << 16);
+    unsigned incl = own;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned t = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += t;
+    }
+    const unsigned all = (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+    const unsigned n = all & 0xFFFFu, first = incl - own;
+    if (!all && !full) return;  // the workgroup as a whole
+    if (all >> 16 && threadIdx.x == 0) gbase = atomicAdd(nsrc, all >> 16);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (int row = w; row < RECON_H; row += NW) {
+        const unsigned long long rl = lane_word(wl, row);
+        const unsigned at = (unsigned)__builtin_amdgcn_readlane((int)first, row) & 0xFFFFu;
+        const bool on = rl >> lane & 1ull;
+        if (on) list[at + (unsigned)__popcll(rl & below)] = (unsigned short)(row * 64 + lane);
+        if (full && !on && i0 + lane < G.ni && jb + row < G.nj) {
+            const size_t c = cix(G, i0 + lane + 1, jb + row + 1);
+            O.P.nx[c] = 0.0;
+            O.P.ny[c] = 1.0;
+        }
+    }
+    __syncthreads();
+    if (all >> 16)
+        for (int row = w; row < RECON_H; row += NW) {
+            const unsigned long long rs = lane_word(ws, row);
+            const unsigned at = (unsigned)__builtin_amdgcn_readlane((int)first, row) >> 16;
+            if (rs >> lane & 1ull)
+                srcs[gbase + at + (unsigned)__popcll(rs & below)] = (int)cix(G, i0 + lane + 1, jb + row + 1);
+        }
+    for (unsigned t = threadIdx.x; t < n; t += RECON_NT) {
+        const unsigned e = list[t];
+        const int c = (int)cix(G, i0 + (int)(e & 63u) + 1, jb + (int)(e >> 6) + 1);
+        recon_cell<DIR>(G, vof, phi, O, dtv, c, full != 0);
     }
 }
 
-// One sweep.  IMPL: first sweep of the sub-step (implicit divergence, clip);
-// otherwise second sweep (explicit divergence with the first sweep's
-// tv/tl).  level: Depthw+etau of the west inflow (x sweeps).  Every operand
-// a cell may need is loaded up front, with neighbour indices clamped to the
-// line, before any of them decides which one is used: the upwind choice
-// then costs no second round trip to memory.
-template <bool X, bool IMPL>
-__global__ void __launch_bounds__(256) k_sweep(ClsGeo G, SweepIn s, double dtv, double level,
-                                               const double* __restrict__ tv_in, const double* __restrict__ tl_in,
-                                               double* __restrict__ tv_out, double* __restrict__ tl_out,
-                                               double* __restrict__ vof_out, double* __restrict__ phi_out) {
-    // x sweeps: XCD-aware tiles, so the tiles either side of a tile (whose
-    // cells its stencil reads) share its L2; y sweeps: launch order, which
-    // keeps vertically adjacent tiles on one XCD already
-    int tx = blockIdx.x, ty = blockIdx.y;
-    if (X) xcd_tile(tx, ty);
-    const int i = tx * blockDim.x + threadIdx.x + 1;
-    const int j = ty * blockDim.y + threadIdx.y + 1;
-    if (i > G.ni || j > G.nj) return;
+// The sweep's update of inner cell (i,j): t the new volume fraction (IMPL: the
+// unclipped temvf), q the new level set.  Every operand a cell may need is
+// loaded up front, with neighbour indices clamped to the line, before any of
+// them decides which one is used: the upwind choice then costs no second round
+// trip to memory.  OPEN: the cell and its neighbours along the sweep are free
+// of solid, with open faces (k_open), so the aperture, solid fraction and face
+// flag arrays are not read: their values are those written here.
+//
+// The first and last cells of a line lie on the domain's ring, whose results
+// Boundary_Condition overwrites; so the reference's fluxes through the domain's
+// own faces (the inflow among them) reach no cell and are not worked out.
+template <bool X, bool IMPL, bool OPEN>
+__device__ __forceinline__ void sweep_cell(const ClsGeo& G, const SweepIn& s, double dtv,
+                                           const double* __restrict__ tv_in, int i, int j, double& t, double& q) {
     const Line<X> L{G, X ? j : i};
     const int a = X ? i : j;
     const int n = L.na();
-    const int am1 = a > 1 ? a - 1 : a, am2 = a > 2 ? a - 2 : am1;
-    const int ap1 = a < n ? a + 1 : a, ap2 = a + 1 < n ? a + 2 : ap1;
-    const size_t c = L.c(a), cm = L.c(am1), cp = L.c(ap1);
-    const double vs = G.vofS[c], vsm = G.vofS[cm], vsp = G.vofS[cp];
+    const int am2 = a > 2 ? a - 2 : a - 1;
+    const int ap2 = a + 1 < n ? a + 2 : a + 1;
+    const size_t c = L.c(a), cm = L.c(a - 1), cp = L.c(a + 1);
+    const double vs = OPEN ? 0.0 : G.vofS[c], vsm = OPEN ? 0.0 : G.vofS[cm], vsp = OPEN ? 0.0 : G.vofS[cp];
     const double f0 = s.vof[c], fm = s.vof[cm], fp = s.vof[cp];
-    const double wm = L.vel(a - 1), w0 = L.vel(a);
-    const double am0 = L.am(a), ap0 = L.ap(a), apm = L.ap(am1), amp = L.am(ap1);
+    const double wm = OPEN ? L.raw(a - 1) : L.vel(a - 1), w0 = OPEN ? L.raw(a) : L.vel(a);
+    const double am0 = OPEN ? 1.0 : L.am(a), ap0 = OPEN ? 1.0 : L.ap(a);
+    const double apm = OPEN ? 1.0 : L.ap(a - 1), amp = OPEN ? 1.0 : L.am(a + 1);
     const double ph0 = s.phi[c], phm1 = s.phi[cm], php1 = s.phi[cp];
     const double phm2 = s.phi[L.c(am2)], php2 = s.phi[L.c(ap2)];
     const double h = L.h(a);
-    double tvi = 0.0, tli = 0.0;
-    if (!IMPL) {
-        tvi = tv_in[c];
-        tli = tl_in[c];
-    }
+    const double tvi = IMPL ? 0.0 : tv_in[c];
     // volume of fluid: temvf(a) after the sweep's in-place updates
-    double t = f0;
+    t = f0;
     if (vs < 1.0 - VOFEPS) t = t / (1.0 - vs);
-    if (a >= 2) {
+    {
         // face a-1: upwind cell a-1 or a
         const double fx = (X ? (wm >= 0.0) : (wm > 0.0)) ? upwind_flux(wm, fm, vsm, apm, s.fr, cm, dtv)
                                                          : upwind_flux(wm, f0, vs, am0, s.fl, c, dtv);
         t = t * (1.0 - vs) + fx * am0 / h;
     }
     {
-        // face a: upwind cell a or a+1; the last face takes cell a's vof
-        double fx;
-        if (X ? (w0 >= 0.0) : (w0 > 0.0))
-            fx = upwind_flux(w0, f0, vs, ap0, s.fr, c, dtv);
-        else if (a < n)
-            fx = upwind_flux(w0, fp, vsp, amp, s.fl, cp, dtv);
-        else
-            fx = f0 * w0 * dtv;
+        // face a: upwind cell a or a+1
+        const double fx = (X ? (w0 >= 0.0) : (w0 > 0.0)) ? upwind_flux(w0, f0, vs, ap0, s.fr, c, dtv)
+                                                         : upwind_flux(w0, fp, vsp, amp, s.fl, cp, dtv);
         t = t - fx * ap0 / h;
     }
-    if (a == 1) {
-        double fin = 0.0;
-        if (X) {
-            if (G.yc[j - 1] - G.dy[j - 1] / 2.0 < level) fin = f0 * wm * dtv;
-        } else {
-            fin = f0 * wm * dtv;
-        }
-        t = t + fin * L.am(1) / L.h(1);
-    }
     // level set: temls(a)
-    double q = ph0;
-    if (a >= 3) q = q * (1.0 - vs) + ls_face(wm, a - 1, n, phm2, phm1, ph0, php1, dtv) * am0 / h;
-    if (a >= 2 && a <= n - 1) q = q - ls_face(w0, a, n, phm1, ph0, php1, php2, dtv) * ap0 / h;
-    if (a == 1) {
-        q = q - ls_flux_first<X>(L, s.phi, dtv) * L.ap(1) / L.h(1);
-        q = q + ph0 * wm * dtv * L.am(1) / L.h(1);
-    }
-    if (a == 2) q = q + ls_flux_first<X>(L, s.phi, dtv) * L.ap(1) / L.h(2);
-    if (a == n) {
-        const double fl = ls_flux_last<X>(L, s.phi, dtv);
-        q = X ? q - fl * L.ap(n) / L.h(n) : q - fl / L.h(n);
-    }
+    q = ph0;
+    if (OPEN || a >= 3) q = q * (1.0 - vs) + ls_face(wm, a - 1, n, phm2, phm1, ph0, php1, dtv) * am0 / h;
+    q = q - ls_face(w0, a, n, phm1, ph0, php1, php2, dtv) * ap0 / h;
+    if (!OPEN && a == 2) q = q + ls_flux_first<X>(L, s.phi, dtv) * L.ap(1) / L.h(2);
     const double dvel = w0 * ap0 - wm * am0;
     if (IMPL) {
         const double den = (1.0 - vs + TOLDENO) - dtv / h * dvel;
         t = t / den;
         q = q / den;
-        tv_out[c] = t;
-        tl_out[c] = q;
-        double f = t * (1.0 - vs);
-        if (f >= 1.0 - VOFEPS - vs) f = 1.0 - vs;
-        if (f < VOFEPS) f = 0.0;
+    } else {
+        // ph0 is the first sweep's temls: only the ring's was overwritten
+        t = t + dtv / h * tvi * dvel;
+        q = q + dtv / h * ph0 * dvel;
+        q = vs < 1.0 - EPSI ? q / (1.0 - vs) : ph0;
+    }
+}
+
+// One sweep with its boundary copy (Boundary_Condition :961-973): every thread
+// works out an inner cell, a thread of the domain's ring the one its cell
+// copies.  IMPL: first sweep of the sub-step (implicit divergence, clip);
+// otherwise second sweep (explicit divergence with the first sweep's temvf).
+// The results' class bits go out with them: a wavefront covers 32 cells of two
+// rows, half a word each.
+//
+// Bound by bytes: 48 a cell in an open tile (vof, phi, a velocity, and three
+// written, or temvf and two written), 76 otherwise.  At 2048^2 an x sweep takes
+// 54 us (3.7 TB/s on the 48), a y sweep, whose halo rows are read again, 60 to
+// 69 us; with a temls array of its own, the arrays above read everywhere and
+// the boundary copy in a launch of its own, 74 to 80 us and 4.9 for the copy.
+constexpr int SWEEP_W = 32, SWEEP_H = 8;  // cells per workgroup (a word half: SWEEP_W = 32)
+template <bool X, bool IMPL>
+__global__ void __launch_bounds__(SWEEP_W * SWEEP_H) k_sweep(ClsGeo G, SweepIn s, Bits B, double dtv,
+                                                             const unsigned char* __restrict__ open,
+                                                             const double* __restrict__ tv_in,
+                                                             double* __restrict__ tv_out,
+                                                             double* __restrict__ vof_out,
+                                                             double* __restrict__ phi_out) {
+    // x sweeps: XCD-aware tiles, so the tiles either side of a tile (whose
+    // cells its stencil reads) share its L2; y sweeps: launch order, which
+    // keeps vertically adjacent tiles on one XCD already
+    int tx = blockIdx.x, ty = blockIdx.y;
+    if (X) xcd_tile(tx, ty);
+    const int i = tx * SWEEP_W + threadIdx.x + 1;
+    const int j = ty * SWEEP_H + threadIdx.y + 1;
+    const bool in = i <= G.ni && j <= G.nj;
+    const bool free = open && (open[(size_t)ty * gridDim.x + tx] >> (X ? 0 : 1) & 1);
+    double f = 0.0, q = 0.0, vs = 0.0;
+    if (in) {
+        // the inner cell whose result this cell takes
+        const int si = min(max(i, 2), G.ni - 1), sj = min(max(j, 2), G.nj - 1);
+        const size_t c = cix(G, i, j);
+        double t;
+        if (free) {
+            sweep_cell<X, IMPL, true>(G, s, dtv, tv_in, si, sj, t, q);
+        } else {
+            vs = G.vofS[c];
+            sweep_cell<X, IMPL, false>(G, s, dtv, tv_in, si, sj, t, q);
+        }
+        f = t;
+        if (IMPL) {
+            tv_out[c] = t;
+            const double vss = free ? 0.0 : G.vofS[cix(G, si, sj)];
+            f = t * (1.0 - vss);
+            if (f >= 1.0 - VOFEPS - vss) f = 1.0 - vss;
+            if (f < VOFEPS) f = 0.0;
+        }
         vof_out[c] = f;
         phi_out[c] = q;
-    } else {
-        t = t + dtv / h * tvi * dvel;
-        q = q + dtv / h * tli * dvel;
-        vof_out[c] = t;
-        phi_out[c] = vs < 1.0 - EPSI ? q / (1.0 - vs) : ph0;
     }
+    unsigned long long b[NBITS];
+    b[BIT_LIST] = __ballot(in && bit_list(f, vs));
+    if (!IMPL) {
+        b[BIT_SRC] = __ballot(in && bit_src(f, vs));
+        b[BIT_GAS] = __ballot(in && bit_gas(f));
+        b[BIT_LIQ] = __ballot(in && bit_liq(f, vs));
+    }
+    if (threadIdx.x < (IMPL ? 1 : NBITS) && j <= G.nj) {
+        const int k = threadIdx.x;
+        const unsigned long long v =
+            IMPL || k == 0 ? b[BIT_LIST] : k == 1 ? b[BIT_SRC] : k == 2 ? b[BIT_GAS] : b[BIT_LIQ];
+        ((unsigned*)B.w[k])[(size_t)(j - 1) * (2 * B.mw) + tx] = (unsigned)(v >> (threadIdx.y % 2 * 32));
+    }
+}
+
+// The sweep tiles free of solid: bit 0 (1) when no cell of the tile or beside it
+// along x (y) holds solid or has a face along x (y) that is masked or not fully
+// open, and the tile does not touch the domain's ring.  Once per call, since
+// every sweep of a call sees the same geometry unless the solid moves.
+// Bound by its 48 bytes a cell: a workgroup takes OPEN_TILES tiles of a column
+// of them with every load issued before the first test (57.8 us at 2048^2, 71.6
+// with one tile a workgroup).
+constexpr int OPEN_TILES = 4;
+__global__ void __launch_bounds__(SWEEP_W * SWEEP_H) k_open(ClsGeo G, unsigned char* __restrict__ open, int nty) {
+    __shared__ unsigned closed[OPEN_TILES];
+    const int x = threadIdx.x, y = threadIdx.y;
+    const int i0 = blockIdx.x * SWEEP_W, t0 = blockIdx.y * OPEN_TILES;
+    if (y == 0 && x < OPEN_TILES) closed[x] = 0u;
+    __syncthreads();
+    unsigned bad[OPEN_TILES];
+#pragma unroll
+    for (int k = 0; k < OPEN_TILES; ++k) {
+        const int j0 = (t0 + k) * SWEEP_H;
+        bad[k] = 0u;
+        if (i0 == 0 || j0 == 0 || i0 + SWEEP_W >= G.ni || j0 + SWEEP_H >= G.nj) {
+            bad[k] = 3u;
+            continue;
+        }
+        auto check = [&](int i, int j, unsigned dirs) {
+            const size_t c = cix(G, i, j), g = gix(G, i, j);
+            const bool e = G.vofS[c] == 0.0;
+            unsigned b = 0u;
+            if (dirs & 1u) b |= !(e & (G.aE[g] == 1.0) & (G.aW[g] == 1.0) & (G.uflag[c] != 0)) ? 1u : 0u;
+            if (dirs & 2u) b |= !(e & (G.aN[g] == 1.0) & (G.aS[g] == 1.0) & (G.vflag[c] != 0)) ? 2u : 0u;
+            return b;
+        };
+        bad[k] = check(i0 + x + 1, j0 + y + 1, 3u);
+        if (x < 2) bad[k] |= check(x ? i0 + SWEEP_W + 1 : i0, j0 + y + 1, 1u);
+        if (y < 2) bad[k] |= check(i0 + x + 1, y ? j0 + SWEEP_H + 1 : j0, 2u);
+    }
+#pragma unroll
+    for (int k = 0; k < OPEN_TILES; ++k)
+        if (bad[k]) atomicOr(&closed[k], bad[k]);
+    __syncthreads();
+    if (y == 0 && x < OPEN_TILES && t0 + x < nty)
+        open[(size_t)(t0 + x) * gridDim.x + blockIdx.x] = (unsigned char)(~closed[x] & 3u);
 }
 
 // ---- redistance -----------------------------------------------------------------
@@ -1196,8 +1266,8 @@ struct PairView {
 // Each pair proposes a distance to its target; two- and three-phase
 // targets keep the minimum (the bit pattern of a non-negative double orders
 // like the value).  Full-solid targets are left to the ordered gather of
-// k_redistance_band.  `best` and `hit` hold +inf and 0 on entry: every cell
-// a pair can reach lies in the band, and k_redistance_band puts them back
+// k_redistance.  `best` and `hit` hold +inf and 0 on entry: every cell
+// a pair can reach lies in the band, and k_redistance puts them back
 // after reading them.
 __global__ void __launch_bounds__(256) k_rd_scatter(ClsGeo G, const double* __restrict__ vof,
                                                     const double* __restrict__ phi, Planes P, PairView pv,
@@ -1233,143 +1303,126 @@ __global__ void __launch_bounds__(256) k_rd_scatter(ClsGeo G, const double* __re
     }
 }
 
-// The band bitmap of k_redistance: word (w, j) is nonzero when an interface
-// cell lies in rows j-BAND..j+BAND of mask words w-1..w+1, a superset of the
-// windows of the 64 cells of word (w, j) (BAND < 64)
-__global__ void __launch_bounds__(256) k_rd_dilate(int nj, int mw, const unsigned long long* __restrict__ mask,
-                                                   unsigned long long* __restrict__ dil, int* __restrict__ band,
-                                                   unsigned* __restrict__ nband) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= mw * nj) return;
-    const int w = k % mw, j = k / mw;
-    unsigned long long any = 0ull;
-    for (int r = max(j - BAND, 0); r <= min(j + BAND, nj - 1); ++r) {
-        const unsigned long long* row = mask + (size_t)r * mw;
-        any |= row[w];
-        if (w > 0) any |= row[w - 1];
-        if (w + 1 < mw) any |= row[w + 1];
-    }
-    dil[k] = any;
-    if (any) band[atomicAdd(nband, 1u)] = k;
+// bits lane-BAND .. lane+BAND of a row's words l, m, r (bit k <-> column
+// offset k - BAND from the lane's cell)
+__device__ __forceinline__ unsigned window_bits(unsigned long long l, unsigned long long m, unsigned long long r,
+                                                int lane) {
+    const int lo = lane - BAND;
+    unsigned long long b = lo >= 0 ? m >> lo : (m << -lo) | (l >> (64 + lo));
+    if (lo > 64 - (2 * BAND + 1)) b |= r << (64 - lo);
+    return (unsigned)b & ((1u << (2 * BAND + 1)) - 1u);
 }
 
-// Redistance, per cell: interface cells take their plane constant, cells
-// reached from an interface cell the nearest distance, the rest the band
-// value.  Full-solid targets replay their visits in the reference's source
-// order (i ascending, then j ascending).  `near`: the cell's band bitmap
-// word is nonzero (else no interface cell lies in its window).
-__device__ void redistance_cell(const ClsGeo& G, const double* __restrict__ vof, const Planes& P,
-                                const unsigned long long* __restrict__ mask, int mw,
-                                const unsigned long long* __restrict__ best, const unsigned char* __restrict__ hit,
-                                double* __restrict__ phi, int ti, int tj, bool near) {
-    const size_t c = cix(G, ti, tj);
-    Target T;
-    T.v = vof[c];
-    T.s = G.vofS[c];
-    // the scatter's minimum and hit flag, loaded with the cell's own data
-    // rather than after the window scan that decides whether they are used
-    const unsigned long long bc = best[c];
-    const bool hc = hit[c] != 0;
-    const double hy = G.dy[tj - 1];
-    if (rd_source(T.v, T.s)) {
-        double n1, n2, d1;
-        plane_of(G, P, c, T.v, hy, n1, n2, d1);
-        phi[c] = d1;  // an interface cell keeps its own plane constant
-        return;
+// Redistance over the grid, one wavefront per 64-cell word of the source mask:
+// interface cells take their plane constant, cells reached from an interface
+// cell the nearest distance, the rest the band value.
+//
+// A word is in the band when an interface cell lies in rows j-BAND..j+BAND of
+// mask words w-1..w+1, a superset of the windows of its 64 cells (BAND < 64).
+// The wavefront reads those 27 words once, one per lane; or-ed over the rows
+// they say of every lane whether its window holds a source.  In the band each
+// cell's minimum and hit flag go back to +inf and 0 once read, ready for the
+// next k_rd_scatter: the band holds every cell a pair can reach.  Full-solid
+// targets replay their visits in the reference's source order (i ascending,
+// then j ascending).
+//
+// Bound by its bytes, 8 a cell outside the band and 33 to 50 inside, and on a
+// small grid by two trips to memory.  One kernel, because as three (test and
+// list the words, cells outside, cells inside) it took 13.8 us at 333 x 171 and
+// 69 us at 2048^2, against 4.2 and 31.2 us.
+__global__ void __launch_bounds__(256) k_redistance(ClsGeo G, const double* __restrict__ vof, Planes P, Bits B,
+                                                    unsigned long long* __restrict__ best,
+                                                    unsigned char* __restrict__ hit, double* __restrict__ phi) {
+    constexpr int ROWS = 2 * BAND + 1;
+    const unsigned long long* mask = B.w[BIT_SRC];
+    const int mw = B.mw;
+    const int lane = threadIdx.x & 63;
+    const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (k >= mw * G.nj) return;  // the wavefront as a whole
+    const int w = k % mw, tj = k / mw + 1, ti = w * 64 + lane + 1;
+    const bool in = ti <= G.ni;
+    const size_t c = cix(G, in ? ti : G.ni, tj);
+    unsigned long long bits = 0ull;
+    {
+        const int r = tj - 1 + (lane & 15) - BAND, x = w + (lane >> 4) - 1;
+        if ((lane & 15) < ROWS && lane < 48 && r >= 0 && r < G.nj && x >= 0 && x < mw)
+            bits = mask[(size_t)r * mw + x];
     }
-    double pa = 1.0e4;
-    bool visited = false;
-    if (rd_target(T.v, T.s) && near) {
-        const int ilo = max(ti - BAND, 1), ihi = min(ti + BAND, G.ni);
-        const int jlo = max(tj - BAND, 1), jhi = min(tj + BAND, G.nj);
-        // window bits per row: bit k <-> source column ilo+k
-        unsigned rows[2 * BAND + 1];
-        unsigned any = 0;
-        for (int sj = jlo; sj <= jhi; ++sj) {
-            const unsigned long long* r = mask + (size_t)(sj - 1) * mw;
-            const int b0 = ilo - 1, w0 = b0 >> 6, w1 = (ihi - 1) >> 6, sh = b0 & 63;
-            unsigned long long bits = r[w0] >> sh;
-            if (w1 != w0 && sh) bits |= r[w1] << (64 - sh);
-            const unsigned win = (unsigned)(bits & ((1ull << (ihi - ilo + 1)) - 1ull));
-            rows[sj - jlo] = win;
-            any |= win;
+    const unsigned long long gas = B.w[BIT_GAS][k], liq = B.w[BIT_LIQ][k];
+    const double hx = G.dx[(in ? ti : G.ni) - 1], hy = G.dy[tj - 1];
+    unsigned long long any = bits;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) any |= __shfl_xor(any, o, 64);
+    const unsigned long long l = lane_word(any, 0), m = lane_word(any, 16), r = lane_word(any, 32);
+    if (l | m | r) {
+        Target T;
+        T.v = vof[c];
+        T.s = G.vofS[c];
+        const unsigned long long bc = best[c];
+        const bool hc = hit[c] != 0;
+        const bool source = rd_source(T.v, T.s);
+        const bool visited = in && !source && rd_target(T.v, T.s) && window_bits(l, m, r, lane);
+        double pa = 1.0e4;
+        if (in && bc != BEST_NONE) best[c] = BEST_NONE;
+        if (in && hc) hit[c] = 0;
+        if (in && source) {
+            double n1, n2, d1;
+            plane_of(G, P, c, T.v, hy, n1, n2, d1);
+            phi[c] = d1;  // an interface cell keeps its own plane constant
         }
-        visited = any != 0;
-        if (visited) {
-            if (T.s >= 1.0 - EPSI) {
+        const bool solid = T.s >= 1.0 - EPSI;
+        if (visited && !solid) {
+            const double b = __longlong_as_double((long long)bc);
+            if (T.s < EPSI) {
+                if (hc) pa = fsign(1.0, 0.5 - T.v) * fmin(b, 1.0e4);
+            } else if (b < 1.0e4) {
+                pa = T.v >= 1.0 - VOFEPS - T.s ? -b : b;
+            }
+        }
+        if (__ballot(visited && solid)) {
+            // the sources of the window, column by column: bit ROWS * column + row
+            unsigned long long set[2] = {0ull, 0ull};
+#pragma unroll
+            for (int row = 0; row < ROWS; ++row) {
+                const unsigned win = window_bits(lane_word(bits, row), lane_word(bits, 16 + row),
+                                                 lane_word(bits, 32 + row), lane);
+#pragma unroll
+                for (int col = 0; col < ROWS; ++col) {
+                    const int at = ROWS * col + row;
+                    set[at >> 6] |= (unsigned long long)(win >> col & 1u) << (at & 63);
+                }
+            }
+            if (visited && solid) {
                 T.phi = phi[c];
                 T.x = G.xc[ti - 1];
                 T.y = G.yc[tj - 1];
-                for (int si = ilo; si <= ihi; ++si) {
-                    for (int sj = jlo; sj <= jhi; ++sj) {
-                        if (!((rows[sj - jlo] >> (si - ilo)) & 1u)) continue;
-                        const size_t sc = cix(G, si, sj);
-                        double n1, n2, d1;
-                        plane_of(G, P, sc, vof[sc], G.dy[sj - 1], n1, n2, d1);
-                        apply(propose(src_cell(G, si, sj), ti - si, tj - sj, n1, n2, d1, T), T, pa);
+                while (set[0] | set[1]) {
+                    int at;
+                    if (set[0]) {
+                        at = __ffsll((long long)set[0]) - 1;
+                        set[0] &= set[0] - 1ull;
+                    } else {
+                        at = 64 + __ffsll((long long)set[1]) - 1;
+                        set[1] &= set[1] - 1ull;
                     }
-                }
-            } else {
-                const double b = __longlong_as_double((long long)bc);
-                if (T.s < EPSI) {
-                    if (hc) pa = fsign(1.0, 0.5 - T.v) * fmin(b, 1.0e4);
-                } else if (b < 1.0e4) {
-                    pa = T.v >= 1.0 - VOFEPS - T.s ? -b : b;
+                    const int ii = at / ROWS - BAND, jj = at % ROWS - BAND;  // source - target
+                    const int si = ti + ii, sj = tj + jj;
+                    const size_t sc = cix(G, si, sj);
+                    double n1, n2, d1;
+                    plane_of(G, P, sc, vof[sc], G.dy[sj - 1], n1, n2, d1);
+                    apply(propose(src_cell(G, si, sj), -ii, -jj, n1, n2, d1, T), T, pa);
                 }
             }
         }
-    }
-    if (visited && !(pa > 9.999e3)) {
-        phi[c] = pa;
-        return;
-    }
-    const double hx = G.dx[ti - 1];
-    if (T.v <= VOFEPS)
-        phi[c] = (double)(BAND + 1) * sqrt(hx * hx + hy * hy);
-    else if (T.v >= (1.0 - VOFEPS - T.s))
-        phi[c] = -(double)(BAND + 1) * sqrt(hx * hx + hy * hy);
-}
-
-// the cells of the listed band words, one wavefront per word (the window
-// scans and nearest-distance gathers; few words, many registers).  Each
-// cell's minimum and hit flag go back to +inf and 0 once read, ready for
-// the next k_rd_scatter: the band holds every cell a pair can reach.
-__global__ void __launch_bounds__(256) k_redistance_band(ClsGeo G, const double* __restrict__ vof, Planes P,
-                                                         const unsigned long long* __restrict__ mask, int mw,
-                                                         const int* __restrict__ band,
-                                                         const unsigned* __restrict__ nband,
-                                                         unsigned long long* __restrict__ best,
-                                                         unsigned char* __restrict__ hit,
-                                                         double* __restrict__ phi) {
-    const unsigned n = *nband;
-    const int lane = threadIdx.x & 63;
-    for (unsigned e = blockIdx.x * 4 + (threadIdx.x >> 6); e < n; e += gridDim.x * 4) {
-        const int k = band[e];
-        const int ti = (k % mw) * 64 + lane + 1, tj = k / mw + 1;
-        if (ti <= G.ni) {
-            redistance_cell(G, vof, P, mask, mw, best, hit, phi, ti, tj, true);
-            const size_t c = cix(G, ti, tj);
-            best[c] = BEST_NONE;
-            hit[c] = 0;
+        if (!in || source) return;
+        if (visited && !(pa > 9.999e3)) {
+            phi[c] = pa;
+            return;
         }
     }
-}
-
-// every other cell: no interface cell in its window, so it takes the band
-// value (or keeps its own level set), with the occupancy of a light kernel
-__global__ void __launch_bounds__(256) k_redistance_far(ClsGeo G, const double* __restrict__ vof,
-                                                        const unsigned long long* __restrict__ dil, int mw,
-                                                        double* __restrict__ phi) {
-    const int ti = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int tj = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    if (ti > G.ni || tj > G.nj) return;
-    if (dil[(size_t)(tj - 1) * mw + ((ti - 1) >> 6)] != 0ull) return;
-    const size_t c = cix(G, ti, tj);
-    const double v = vof[c], s = G.vofS[c];
-    const double hx = G.dx[ti - 1], hy = G.dy[tj - 1];
-    if (v <= VOFEPS)
+    if (gas >> lane & 1ull)  // (no bit beyond the grid)
         phi[c] = (double)(BAND + 1) * sqrt(hx * hx + hy * hy);
-    else if (v >= (1.0 - VOFEPS - s))
+    else if (liq >> lane & 1ull)
         phi[c] = -(double)(BAND + 1) * sqrt(hx * hx + hy * hy);
 }
 
@@ -1559,8 +1612,6 @@ int clsvof_allocate(Ctx* c) {
     B.vt = (double*)dev_alloc(c, n * sizeof(double));
     B.pt = (double*)dev_alloc(c, n * sizeof(double));
     B.tv = (double*)dev_alloc(c, n * sizeof(double));
-    B.tl = (double*)dev_alloc(c, n * sizeof(double));
-    B.stale = (unsigned char*)dev_alloc(c, n);
     B.hit = (unsigned char*)dev_alloc(c, n);
     B.best = (unsigned long long*)dev_alloc(c, n * sizeof(unsigned long long));
     if (B.best) {
@@ -1569,16 +1620,13 @@ int clsvof_allocate(Ctx* c) {
         if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) return SG_ERR_ALLOC;
     }
     B.srcs = (int*)dev_alloc(c, n * sizeof(int));
-    B.stales = (int*)dev_alloc(c, n * sizeof(int));
-    B.ifc = (int*)dev_alloc(c, n * sizeof(int));
     B.fr = (double*)dev_alloc(c, n * sizeof(double));
     B.fl = (double*)dev_alloc(c, n * sizeof(double));
-    B.cnt = (unsigned*)dev_alloc(c, ClsBuffers::CNT_SLOTS * sizeof(unsigned));
-    B.mask = (unsigned long long*)dev_alloc(c, (size_t)B.mw * c->nj * sizeof(unsigned long long));
-    B.dil = (unsigned long long*)dev_alloc(c, (size_t)B.mw * c->nj * sizeof(unsigned long long));
-    B.band = (int*)dev_alloc(c, (size_t)B.mw * c->nj * sizeof(int));
-    if (!B.xc || !B.yc || !B.dis || !B.vt || !B.pt || !B.tv || !B.tl || !B.stale || !B.hit || !B.best || !B.srcs ||
-        !B.stales || !B.ifc || !B.fr || !B.fl || !B.cnt || !B.mask || !B.dil || !B.band)
+    B.cnt = (unsigned*)dev_alloc(c, ClsBuffers::MAX_NSUB * sizeof(unsigned));
+    B.bits = (unsigned long long*)dev_alloc(c, NBITS * (size_t)B.mw * c->nj * sizeof(unsigned long long));
+    B.open = (unsigned char*)dev_alloc(c, (size_t)((c->ni + SWEEP_W - 1) / SWEEP_W) * ((c->nj + SWEEP_H - 1) / SWEEP_H));
+    if (!B.xc || !B.yc || !B.dis || !B.vt || !B.pt || !B.tv || !B.hit || !B.best || !B.srcs || !B.fr || !B.fl ||
+        !B.cnt || !B.bits || !B.open)
         return SG_ERR_ALLOC;
     return SG_OK;
 }
@@ -1597,54 +1645,67 @@ int sweep_timing_drain(Ctx* c) {
     return SG_OK;
 }
 
+// From how many cells a call works out which of its sweep tiles are free of
+// solid.  Measured on a whole call of 6 sub-steps (12 sweeps) with and without:
+// at 2048^2, where a sweep is bound by its bytes, 1498 against 1612 us; at 1024^2,
+// 768^2 and 512^2, where its arrays stay in the last-level cache, 641 against 640,
+// 586 against 585 and 508 against 491 us.  Their 3 arrays of results and 3 of
+// operands outgrow that cache's 256 MB together with the geometry between the two.
+constexpr size_t OPEN_MIN_CELLS = 1ull << 21;
+
 // Coupled_LS_VOF on the device fields VOF, PHI (in/out), NX, NY (out),
-// U, V (in).  `levels` holds Depthw+etau of each sub-step.
-int clsvof_advect(Ctx* c, double dt, int nsub, const double* levels) {
+// U, V (in).
+int clsvof_advect(Ctx* c, double dt, int nsub) {
     const ClsGeo G = make_geo(c);
     ClsBuffers& B = c->cls;
     double* vof = (double*)c->field[SG_F_VOF];
     double* phi = (double*)c->field[SG_F_PHI];
     const Planes P{(double*)c->field[SG_F_NX], (double*)c->field[SG_F_NY], B.dis};
-    const dim3 blk(64, 4), grd((c->ni + 63) / 64, (c->nj + 3) / 4);
     const int ring = 2 * c->ni + 2 * (c->nj - 2);
     const dim3 rblk(256), rgrd((ring + 255) / 256);
-    const dim3 pblk(256), pgrd(1024);  // grid-stride loops over the listed pairs / cells
-    const dim3 rcblk(64, RECON_TY),
-        rcgrd((c->ni + 63) / 64, (c->nj + RECON_TY * RECON_R - 1) / (RECON_TY * RECON_R));
+    const dim3 pblk(256), pgrd(1024);  // a grid-stride loop over the listed pairs
+    const dim3 rcgrd((c->ni + 63) / 64, (c->nj + RECON_H - 1) / RECON_H);
     // sweeps: 32x8 tiles (3% faster per transport call than 64x4, 256x1 or
     // 128x2 at 2048^2: the y stencil's rows stay within fewer tiles)
-    const dim3 sblk(32, 8), sgrd((c->ni + 31) / 32, (c->nj + 7) / 8);
+    const dim3 sblk(SWEEP_W, SWEEP_H), sgrd((c->ni + SWEEP_W - 1) / SWEEP_W, (c->nj + SWEEP_H - 1) / SWEEP_H);
     const double dtv = dt / (double)nsub;
     hipStream_t st = c->stream;
-    // three counters per reconstruction, three reconstructions per sub-step,
-    // then one band-word count per sub-step
-    const int slots = 10 * nsub;
-    if (slots > ClsBuffers::CNT_SLOTS) {
+    if (nsub > ClsBuffers::MAX_NSUB) {
         set_error("clsvof_advect: too many sub-steps");
         return SG_ERR_ARG;
     }
-    hipLaunchKernelGGL(k_zero, dim3((slots + 255) / 256), dim3(256), 0, st, B.cnt, slots);
-    int slot = 0;
-    // `scan`: the interface list of the last full-grid scan, when vof and
-    // vofS have not changed since (re-distancing changes phi only)
-    // last: the sub-step's final reconstruction (re-distancing sources);
-    // full: also n = (0,1) on the other cells -- only the transport's very
-    // last one, since within the transport a stored plane is read only
-    // where the cell is an interface cell of the current vof (plane_of,
-    // plane_pick), and every such plane is rewritten by k_recon_ifc
-    auto recon = [&](const double* v, const double* p, bool last, const unsigned* scan, bool full) {
-        unsigned* cnt = B.cnt + slot;
-        slot += 3;
-        if (!scan)
-            hipLaunchKernelGGL(k_recon, rcgrd, rcblk, 0, st, G, v, P, full ? 1 : 0,
-                               last ? B.mask : (unsigned long long*)nullptr, B.mw, B.srcs, B.ifc, cnt);
-        const unsigned* nifc = scan ? scan + 2 : cnt + 2;
-        hipLaunchKernelGGL(k_recon_ifc, dim3(256), pblk, 0, st, G, v, p, P, B.stale, B.ifc, nifc, B.stales, cnt);
-        hipLaunchKernelGGL(k_dis_fix, dim3(64), pblk, 0, st, G, v, B.stale, B.stales, cnt, B.dis);
-        // the interface count (entry 2) the flux precomputation reads
-        return scan ? scan : (const unsigned*)cnt;
+    // the number of sources listed, one per sub-step
+    hipLaunchKernelGGL(k_zero, dim3((nsub + 255) / 256), dim3(256), 0, st, B.cnt, nsub);
+    Bits bits;
+    bits.mw = B.mw;
+    for (int k = 0; k < NBITS; ++k) bits.w[k] = B.bits + (size_t)k * B.mw * c->nj;
+    const bool moves = c->moving.shape.kind != SG_SOLID_NONE;
+    const unsigned char* open = nullptr;
+    if (!moves && (size_t)c->ni * c->nj >= OPEN_MIN_CELLS) {
+        hipLaunchKernelGGL(k_open, dim3(sgrd.x, (sgrd.y + OPEN_TILES - 1) / OPEN_TILES), sblk, 0, st, G, B.open,
+                           (int)sgrd.y);
+        open = B.open;
+    }
+    // One reconstruction and, with `dir`, the face fluxes of the sweep after it.
+    // scan: the class bits are not those of v yet; full: also n = (0,1) on the
+    // other cells -- only the transport's very last one, since within the
+    // transport a stored plane is read only where the cell is an interface cell
+    // of the current vof (plane_of, plane_pick), and every such plane is
+    // rewritten by the reconstruction
+    auto recon = [&](auto dir, const double* v, const double* p, bool scan, bool full, int* srcs, unsigned* nsrc) {
+        constexpr int DIR = decltype(dir)::value;
+        const ReconOut O{P, B.fr, B.fl};
+        if (scan)
+            hipLaunchKernelGGL((k_recon<DIR, true>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv, full ? 1 : 0,
+                               srcs, nsrc);
+        else
+            hipLaunchKernelGGL((k_recon<DIR, false>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv,
+                               full ? 1 : 0, srcs, nsrc);
     };
-    const unsigned* last_scan = nullptr;  // the previous sub-step's final scan
+    using std::integral_constant;
+    const integral_constant<int, FLUX_NONE> no_flux{};
+    const integral_constant<int, FLUX_X> flux_x{};
+    const integral_constant<int, FLUX_Y> flux_y{};
     // sg_sweep_timing: an event before (end = 0) and after (end = 1) each sweep
     auto& TM = c->sweep_timing;
     if (TM.on && TM.used + 2 * nsub > Ctx::SweepTiming::POOL) {
@@ -1658,40 +1719,37 @@ int clsvof_advect(Ctx* c, double dt, int nsub, const double* levels) {
         return e;
     };
     for (int k = 1; k <= nsub; ++k) {
-        const double level = levels[k - 1];
-        // first sweep: (vof, phi) -> (vt, pt), implicit divergence; vof is
-        // the one the previous sub-step's last reconstruction scanned
-        const unsigned* c1 = recon(vof, phi, false, last_scan, false);
-        const SweepIn s1{vof, phi, P, B.fr, B.fl};
+        // first sweep: (vof, phi) -> (vt, pt), implicit divergence; after the
+        // first sub-step the bits are those of the last reconstruction, and
+        // re-distancing has changed phi only
         if (k % 2 == 1)
-            hipLaunchKernelGGL((k_flux_pre<true>), pgrd, pblk, 0, st, G, s1, dtv, B.ifc, c1, B.fr, B.fl);
+            recon(flux_x, vof, phi, k == 1, false, nullptr, nullptr);
         else
-            hipLaunchKernelGGL((k_flux_pre<false>), pgrd, pblk, 0, st, G, s1, dtv, B.ifc, c1, B.fr, B.fl);
+            recon(flux_y, vof, phi, k == 1, false, nullptr, nullptr);
+        const SweepIn s1{vof, phi, B.fr, B.fl};
         SG_HIP(sweep_mark(0));
         if (k % 2 == 1)
-            hipLaunchKernelGGL((k_sweep<true, true>), sgrd, sblk, 0, st, G, s1, dtv, level, nullptr, nullptr, B.tv,
-                               B.tl, B.vt, B.pt);
+            hipLaunchKernelGGL((k_sweep<true, true>), sgrd, sblk, 0, st, G, s1, bits, dtv, open, nullptr, B.tv, B.vt,
+                               B.pt);
         else
-            hipLaunchKernelGGL((k_sweep<false, true>), sgrd, sblk, 0, st, G, s1, dtv, level, nullptr, nullptr, B.tv,
-                               B.tl, B.vt, B.pt);
+            hipLaunchKernelGGL((k_sweep<false, true>), sgrd, sblk, 0, st, G, s1, bits, dtv, open, nullptr, B.tv, B.vt,
+                               B.pt);
         SG_HIP(sweep_mark(1));
-        hipLaunchKernelGGL(k_bc, rgrd, rblk, 0, st, c->ni, c->nj, B.vt, B.pt);
         // second sweep: (vt, pt) -> (vof, phi), explicit divergence
-        const unsigned* c2 = recon(B.vt, B.pt, false, nullptr, false);
-        const SweepIn s2{B.vt, B.pt, P, B.fr, B.fl};
         if (k % 2 == 1)
-            hipLaunchKernelGGL((k_flux_pre<false>), pgrd, pblk, 0, st, G, s2, dtv, B.ifc, c2, B.fr, B.fl);
+            recon(flux_y, B.vt, B.pt, false, false, nullptr, nullptr);
         else
-            hipLaunchKernelGGL((k_flux_pre<true>), pgrd, pblk, 0, st, G, s2, dtv, B.ifc, c2, B.fr, B.fl);
+            recon(flux_x, B.vt, B.pt, false, false, nullptr, nullptr);
+        const SweepIn s2{B.vt, B.pt, B.fr, B.fl};
         SG_HIP(sweep_mark(0));
         if (k % 2 == 1)
-            hipLaunchKernelGGL((k_sweep<false, false>), sgrd, sblk, 0, st, G, s2, dtv, level, B.tv, B.tl, nullptr,
-                               nullptr, vof, phi);
+            hipLaunchKernelGGL((k_sweep<false, false>), sgrd, sblk, 0, st, G, s2, bits, dtv, open, B.tv, nullptr, vof,
+                               phi);
         else
-            hipLaunchKernelGGL((k_sweep<true, false>), sgrd, sblk, 0, st, G, s2, dtv, level, B.tv, B.tl, nullptr,
-                               nullptr, vof, phi);
+            hipLaunchKernelGGL((k_sweep<true, false>), sgrd, sblk, 0, st, G, s2, bits, dtv, open, B.tv, nullptr, vof,
+                               phi);
         SG_HIP(sweep_mark(1));
-        if (c->moving.shape.kind != SG_SOLID_NONE) {
+        if (moves) {
             // ObjectMovement (Clsvof_Mod.f90:2384-2398) over the sub-step,
             // then SolidVolumeFraction on the P cells (:920-921)
             auto& m = c->moving;
@@ -1701,19 +1759,16 @@ int clsvof_advect(Ctx* c, double dt, int nsub, const double* levels) {
             m.vs = m.vs + m.asy * dtv;
             const int rc = solid_fraction_step(c, &m.shape);
             if (rc) return rc;
+            // the solid has changed vof too
+            hipLaunchKernelGGL(k_bc, rgrd, rblk, 0, st, c->ni, c->nj, vof, phi);
         }
-        hipLaunchKernelGGL(k_bc, rgrd, rblk, 0, st, c->ni, c->nj, vof, phi);
         // reconstruction (full normals out) and re-distancing
-        const unsigned* cnt = recon(vof, phi, true, nullptr, k == nsub);
-        last_scan = cnt;
+        unsigned* cnt = B.cnt + (k - 1);
+        recon(no_flux, vof, phi, moves, k == nsub, B.srcs, cnt);
         const PairView pv{B.srcs, cnt};
         hipLaunchKernelGGL(k_rd_scatter, pgrd, pblk, 0, st, G, vof, phi, P, pv, B.best, B.hit);
-        unsigned* nband = B.cnt + 9 * nsub + (k - 1);
-        hipLaunchKernelGGL(k_rd_dilate, dim3((unsigned)((B.mw * c->nj + 255) / 256)), dim3(256), 0, st, c->nj, B.mw,
-                           (const unsigned long long*)B.mask, B.dil, B.band, nband);
-        hipLaunchKernelGGL(k_redistance_far, grd, blk, 0, st, G, vof, (const unsigned long long*)B.dil, B.mw, phi);
-        hipLaunchKernelGGL(k_redistance_band, dim3(2048), dim3(256), 0, st, G, vof, P, B.mask, B.mw,
-                           (const int*)B.band, (const unsigned*)nband, B.best, B.hit, phi);
+        hipLaunchKernelGGL(k_redistance, dim3((unsigned)((B.mw * c->nj + 3) / 4)), dim3(256), 0, st, G, vof, P,
+                           bits, B.best, B.hit, phi);
     }
     SG_HIP(hipGetLastError());
     return SG_OK;

@@ -149,25 +149,17 @@ struct ClsBuffers {
     double* dis = nullptr;  // PLIC plane constants of the last reconstruction
     double* vt = nullptr;   // vof, phi after the first sweep of a sub-step
     double* pt = nullptr;
-    double* tv = nullptr;   // temvf, temls of the first sweep (explicit term)
-    double* tl = nullptr;
-    unsigned char* stale = nullptr;    // plane constant left unassigned
+    double* tv = nullptr;   // temvf of the first sweep (explicit term)
     unsigned char* hit = nullptr;      // re-distancing: two-phase rule applied
     unsigned long long* best = nullptr;  // re-distancing: nearest distance (bits)
     int* srcs = nullptr;               // listed interface cells (re-distancing sources)
-    int* stales = nullptr;             // listed cells with a stale plane constant
-    int* ifc = nullptr;                // listed interface cells of a reconstruction and the cells
-                                       // whose face fluxes need the PLIC geometry
-    double* fr = nullptr;              // the latter's PLIC flux through the far / near face of a sweep
+    double* fr = nullptr;              // PLIC flux through the far / near face of a sweep, where a cell needs it
     double* fl = nullptr;
-    unsigned* cnt = nullptr;           // list lengths, three per reconstruction
-    static constexpr int CNT_SLOTS = 6 * 1024;
-    unsigned long long* mask = nullptr;  // interface cells, 1 bit per cell
-    // per mask word: any interface cell within the band of its 64 cells
-    // (the OR over rows j-BAND..j+BAND of words w-1..w+1)
-    unsigned long long* dil = nullptr;
-    int* band = nullptr;               // the nonzero words of dil (w + j * mw)
-    int mw = 0;                        // mask words per row
+    static constexpr int MAX_NSUB = 614;
+    unsigned* cnt = nullptr;           // sources listed, one count per sub-step
+    unsigned long long* bits = nullptr;  // the cells' class bits, four planes of mw x nj words
+    unsigned char* open = nullptr;     // sweep tiles free of solid
+    int mw = 0;                        // words per row
     double xw = 0.0;                   // west edge x of the grid (host copy)
     double dx0 = 0.0;                  // width of the first column (host copy)
 };
@@ -392,7 +384,7 @@ int momentum_solve(Ctx* c, const double* m, const double* b, double* x, double t
                    double* relres);
 // interface transport (sg_clsvof.hip)
 int clsvof_allocate(Ctx* c);
-int clsvof_advect(Ctx* c, double dt, int nsub, const double* levels);
+int clsvof_advect(Ctx* c, double dt, int nsub);
 int interface_to_uv(Ctx* c);
 
 void* dev_alloc(Ctx* c, size_t bytes);
