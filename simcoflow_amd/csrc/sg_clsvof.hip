@@ -6,12 +6,11 @@
 //   k_recon      PLIC reconstruction (Interface_Reconstruct :1250-1321): find
 //                the interface cells, then, packed one per lane, their normals,
 //                plane constants and the PLIC face fluxes of the coming sweep
-//                (k_recon_ifc: on the cells the last scan listed)
 //   k_sweep      first sweep, implicit divergence (:798-823 / :862-888), with
 //                the boundary copy (Boundary_Condition :961-973)
 //   k_recon
 //   k_sweep      second sweep, explicit divergence (:834-858 / :898-929)
-//   k_recon (+ interface bit mask and source list)
+//   k_recon (+ source list)
 //   k_rd_scatter, k_redistance: level set from the PLIC segments (Redistance
 //                :1525-1708)
 //
@@ -274,6 +273,44 @@ struct PhiView {
     __device__ double Y(int j) const { return G.yc[j - 1]; }
 };
 
+// The level set and the cell centres around an inner cell that its normal may
+// ask for, loaded together before the first test: offsets are compile-time
+// constants, so all of it stays in registers.  Two cells away is clamped to the
+// grid; normal_irre does not use what lies beyond it.
+struct Stencil {
+    double v[13], x[5], y[5];
+    static constexpr int at(int di, int dj) {
+        return dj == 0 ? di + 2 : di == 0 ? 5 + (dj < 0 ? dj + 2 : dj + 1) : 9 + (di > 0 ? 1 : 0) + (dj > 0 ? 2 : 0);
+    }
+    __device__ __forceinline__ double operator()(int di, int dj) const { return v[at(di, dj)]; }
+    __device__ __forceinline__ double X(int di) const { return x[di + 2]; }
+    __device__ __forceinline__ double Y(int dj) const { return y[dj + 2]; }
+};
+__device__ __forceinline__ Stencil stencil(const ClsGeo& G, const double* __restrict__ phi, int i, int j) {
+    Stencil s;
+    const int im = max(i - 2, 1), ip = min(i + 2, G.ni), jm = max(j - 2, 1), jp = min(j + 2, G.nj);
+#pragma unroll
+    for (int d = -1; d <= 1; ++d) {
+        s.v[Stencil::at(d, 0)] = phi[cix(G, i + d, j)];
+        if (d) {
+            s.v[Stencil::at(0, d)] = phi[cix(G, i, j + d)];
+            s.v[Stencil::at(d, -1)] = phi[cix(G, i + d, j - 1)];
+            s.v[Stencil::at(d, 1)] = phi[cix(G, i + d, j + 1)];
+        }
+        s.x[d + 2] = G.xc[i + d - 1];
+        s.y[d + 2] = G.yc[j + d - 1];
+    }
+    s.v[Stencil::at(-2, 0)] = phi[cix(G, im, j)];
+    s.v[Stencil::at(2, 0)] = phi[cix(G, ip, j)];
+    s.v[Stencil::at(0, -2)] = phi[cix(G, i, jm)];
+    s.v[Stencil::at(0, 2)] = phi[cix(G, i, jp)];
+    s.x[0] = G.xc[im - 1];
+    s.x[4] = G.xc[ip - 1];
+    s.y[0] = G.yc[jm - 1];
+    s.y[4] = G.yc[jp - 1];
+    return s;
+}
+
 __device__ __forceinline__ double qual(double vx, double vy) { return fabs(1.0 - sqrt(vx * vx + vy * vy)); }
 
 // The 8 candidate directions of Coupled_LS_VOF (:746-753) as the reference
@@ -288,10 +325,10 @@ __device__ __forceinline__ void vset(int k, double& a, double& b) {
 
 // one-sided pair chosen by the direction most parallel to grad phi
 // (Normal_Vector_Irre :1768-1827 / :1855-1905)
-__device__ void nv_directional(const PhiView& p, int i, int j, int imv0, double& nx, double& ny) {
+__device__ __forceinline__ void nv_directional(const Stencil& p, int imv0, double& nx, double& ny) {
     const double eta = 0.075, nuy = eta / 8.0;
-    const double vx = (p(i + 1, j) - p(i - 1, j)) / (p.X(i + 1) - p.X(i - 1));
-    const double vy = (p(i, j + 1) - p(i, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+    const double vx = (p(1, 0) - p(-1, 0)) / (p.X(1) - p.X(-1));
+    const double vy = (p(0, 1) - p(0, -1)) / (p.Y(1) - p.Y(-1));
     double maxv = 0.0;
     int imv = imv0;
     for (int k = 1; k <= 8; ++k) {
@@ -315,24 +352,24 @@ __device__ void nv_directional(const PhiView& p, int i, int j, int imv0, double&
     }
     double vx1, vx2, vy1, vy2;
     if (v1x == -1.0) {
-        vx1 = (p(i, j) - p(i - 1, j)) / (p.X(i) - p.X(i - 1));
-        vx2 = (p(i + 1, j) - p(i, j)) / (p.X(i + 1) - p.X(i));
+        vx1 = (p(0, 0) - p(-1, 0)) / (p.X(0) - p.X(-1));
+        vx2 = (p(1, 0) - p(0, 0)) / (p.X(1) - p.X(0));
     } else if (v1x == 0.0) {
-        vx1 = (p(i + 1, j) - p(i - 1, j)) / (p.X(i + 1) - p.X(i - 1));
+        vx1 = (p(1, 0) - p(-1, 0)) / (p.X(1) - p.X(-1));
         vx2 = vx1;
     } else {
-        vx1 = (p(i + 1, j) - p(i, j)) / (p.X(i + 1) - p.X(i));
-        vx2 = (p(i, j) - p(i - 1, j)) / (p.X(i) - p.X(i - 1));
+        vx1 = (p(1, 0) - p(0, 0)) / (p.X(1) - p.X(0));
+        vx2 = (p(0, 0) - p(-1, 0)) / (p.X(0) - p.X(-1));
     }
     if (v1y == -1.0) {
-        vy1 = (p(i, j) - p(i, j - 1)) / (p.Y(j) - p.Y(j - 1));
-        vy2 = (p(i, j + 1) - p(i, j)) / (p.Y(j + 1) - p.Y(j));
+        vy1 = (p(0, 0) - p(0, -1)) / (p.Y(0) - p.Y(-1));
+        vy2 = (p(0, 1) - p(0, 0)) / (p.Y(1) - p.Y(0));
     } else if (v1y == 0.0) {
-        vy1 = (p(i, j + 1) - p(i, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+        vy1 = (p(0, 1) - p(0, -1)) / (p.Y(1) - p.Y(-1));
         vy2 = vy1;
     } else {
-        vy1 = (p(i, j + 1) - p(i, j)) / (p.Y(j + 1) - p.Y(j));
-        vy2 = (p(i, j) - p(i, j - 1)) / (p.Y(j) - p.Y(j - 1));
+        vy1 = (p(0, 1) - p(0, 0)) / (p.Y(1) - p.Y(0));
+        vy2 = (p(0, 0) - p(0, -1)) / (p.Y(0) - p.Y(-1));
     }
     if (qual(vx1, vy1) < qual(vx2, vy2) + nuy) {
         nx = vx1;
@@ -343,69 +380,66 @@ __device__ void nv_directional(const PhiView& p, int i, int j, int imv0, double&
     }
 }
 
-// Normal_Vector_Irre (:1710-1919), interior cells
-__device__ void normal_irre(const ClsGeo& G, const double* phi, int i, int j, double& nx, double& ny) {
-    const PhiView p{G, phi};
+// Normal_Vector_Irre (:1710-1919), interior cells; vs the cell's vofS
+__device__ __forceinline__ void normal_irre(const ClsGeo& G, const Stencil& p, double vs, int i, int j, double& nx,
+                                            double& ny) {
     const double eta = 0.075;
-    const double vs = G.vofS[cix(G, i, j)];
     if (vs >= EPSI) {
         const double se = G.vofS[cix(G, i + 1, j)], sw = G.vofS[cix(G, i - 1, j)];
         const double sn = G.vofS[cix(G, i, j + 1)], ss = G.vofS[cix(G, i, j - 1)];
         if (se < 1.0 - EPSI && sw < 1.0 - EPSI)
-            nx = (p(i + 1, j) - p(i - 1, j)) / (p.X(i + 1) - p.X(i - 1));
+            nx = (p(1, 0) - p(-1, 0)) / (p.X(1) - p.X(-1));
         else if (se >= 1.0 - EPSI)
-            nx = (p(i, j) - p(i - 1, j)) / (p.X(i) - p.X(i - 1));
+            nx = (p(0, 0) - p(-1, 0)) / (p.X(0) - p.X(-1));
         else
-            nx = (p(i + 1, j) - p(i, j)) / (p.X(i + 1) - p.X(i));
+            nx = (p(1, 0) - p(0, 0)) / (p.X(1) - p.X(0));
         if (sn < 1.0 - EPSI && ss < 1.0 - EPSI)
-            ny = (p(i, j + 1) - p(i, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+            ny = (p(0, 1) - p(0, -1)) / (p.Y(1) - p.Y(-1));
         else if (sn > 1.0 - EPSI)
-            ny = (p(i, j) - p(i, j - 1)) / (p.Y(j) - p.Y(j - 1));
+            ny = (p(0, 0) - p(0, -1)) / (p.Y(0) - p.Y(-1));
         else
-            ny = (p(i, j + 1) - p(i, j)) / (p.Y(j + 1) - p.Y(j));
+            ny = (p(0, 1) - p(0, 0)) / (p.Y(1) - p.Y(0));
         return;
     }
-    const double cx = (p(i + 1, j) - p(i - 1, j)) / (p.X(i + 1) - p.X(i - 1));
-    const double cy = (p(i, j + 1) - p(i, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+    const double cx = (p(1, 0) - p(-1, 0)) / (p.X(1) - p.X(-1));
+    const double cy = (p(0, 1) - p(0, -1)) / (p.Y(1) - p.Y(-1));
     const double q0 = qual(cx, cy);
     double vx, vy;
-    vx = i >= 3 ? (p(i, j) - p(i - 2, j)) / (p.X(i) - p.X(i - 2)) : (p(i, j) - p(i - 1, j)) / (p.X(i) - p.X(i - 1));
-    vy = (p(i - 1, j + 1) - p(i - 1, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+    vx = i >= 3 ? (p(0, 0) - p(-2, 0)) / (p.X(0) - p.X(-2)) : (p(0, 0) - p(-1, 0)) / (p.X(0) - p.X(-1));
+    vy = (p(-1, 1) - p(-1, -1)) / (p.Y(1) - p.Y(-1));
     const double qm = qual(vx, vy);
-    vx = i <= G.ni - 2 ? (p(i + 2, j) - p(i, j)) / (p.X(i + 2) - p.X(i))
-                       : (p(i + 1, j) - p(i, j)) / (p.X(i + 1) - p.X(i));
-    vy = (p(i + 1, j + 1) - p(i + 1, j - 1)) / (p.Y(j + 1) - p.Y(j - 1));
+    vx = i <= G.ni - 2 ? (p(2, 0) - p(0, 0)) / (p.X(2) - p.X(0))
+                       : (p(1, 0) - p(0, 0)) / (p.X(1) - p.X(0));
+    vy = (p(1, 1) - p(1, -1)) / (p.Y(1) - p.Y(-1));
     const double qp = qual(vx, vy);
-    int sx;
+    int sx = 0, sy = 0;
+    int start = -1;  // the directional rule, and the direction it starts from (one copy of its code)
     if (qm < eta && qp >= eta) sx = -1;
     else if (qm >= eta && qp < eta) sx = 1;
     else if (qm < eta && q0 < eta && qp < eta) sx = 0;
     else if (qm >= eta && q0 >= eta && qp >= eta) sx = 0;
-    else {
-        nv_directional(p, i, j, 0, nx, ny);
-        return;
-    }
-    vy = j >= 3 ? (p(i, j) - p(i, j - 2)) / (p.Y(j) - p.Y(j - 2)) : (p(i, j) - p(i, j - 1)) / (p.Y(j) - p.Y(j - 1));
-    vx = (p(i + 1, j - 1) - p(i - 1, j - 1)) / (p.X(i + 1) - p.X(i - 1));
+    else start = 0;
+    vy = j >= 3 ? (p(0, 0) - p(0, -2)) / (p.Y(0) - p.Y(-2)) : (p(0, 0) - p(0, -1)) / (p.Y(0) - p.Y(-1));
+    vx = (p(1, -1) - p(-1, -1)) / (p.X(1) - p.X(-1));
     const double rm = qual(vx, vy);
-    vx = (p(i + 1, j + 1) - p(i - 1, j + 1)) / (p.X(i + 1) - p.X(i - 1));
-    vy = j <= G.nj - 2 ? (p(i, j + 2) - p(i, j)) / (p.Y(j + 2) - p.Y(j))
-                       : (p(i, j + 1) - p(i, j)) / (p.Y(j + 1) - p.Y(j));
+    vx = (p(1, 1) - p(-1, 1)) / (p.X(1) - p.X(-1));
+    vy = j <= G.nj - 2 ? (p(0, 2) - p(0, 0)) / (p.Y(2) - p.Y(0))
+                       : (p(0, 1) - p(0, 0)) / (p.Y(1) - p.Y(0));
     const double rp = qual(vx, vy);
-    int sy;
     if (rm < eta && rp >= eta) sy = -1;
     else if (rm >= eta && rp < eta) sy = 1;
     else if (rm < eta && q0 < eta && rp < eta) sy = 0;
     else if (rm >= eta && q0 >= eta && rp >= eta) sy = 0;
-    else {
-        nv_directional(p, i, j, 1, nx, ny);
+    else if (start < 0) start = 1;
+    if (start >= 0) {
+        nv_directional(p, start, nx, ny);
         return;
     }
-    if (sx == -1) nx = (p(i, j) - p(i - 1, j)) / (p.X(i) - p.X(i - 1));
-    else if (sx == 1) nx = (p(i + 1, j) - p(i, j)) / (p.X(i + 1) - p.X(i));
+    if (sx == -1) nx = (p(0, 0) - p(-1, 0)) / (p.X(0) - p.X(-1));
+    else if (sx == 1) nx = (p(1, 0) - p(0, 0)) / (p.X(1) - p.X(0));
     else nx = cx;
-    if (sy == -1) ny = (p(i, j) - p(i, j - 1)) / (p.Y(j) - p.Y(j - 1));
-    else if (sy == 1) ny = (p(i, j + 1) - p(i, j)) / (p.Y(j + 1) - p.Y(j));
+    if (sy == -1) ny = (p(0, 0) - p(0, -1)) / (p.Y(0) - p.Y(-1));
+    else if (sy == 1) ny = (p(0, 1) - p(0, 0)) / (p.Y(1) - p.Y(0));
     else ny = cy;
 }
 
@@ -441,18 +475,6 @@ __device__ __forceinline__ double edge_ny(const PhiView& p, int i, int j, int nj
 __device__ __forceinline__ int cls_of(const ClsGeo& G, const double* vof, int i, int j) {
     const size_t c = cix(G, i, j);
     return recon_class(vof[c], G.vofS[c]);
-}
-
-// final normal of an interior cell
-__device__ void final_interior(const ClsGeo& G, const double* vof, const double* phi, int i, int j, double& nx,
-                               double& ny) {
-    if (cls_of(G, vof, i, j)) {
-        normal_irre(G, phi, i, j, nx, ny);
-        normalise(nx, ny);
-    } else {
-        nx = 0.0;
-        ny = 1.0;
-    }
 }
 
 // final normal of a cell on the west or east edge (i = 1 or ni).  Away from
@@ -495,37 +517,48 @@ __device__ void final_side(const ClsGeo& G, const double* vof, const double* phi
     }
 }
 
-// final normal of a cell on the south or north edge (1 < i < ni).  Its x
-// component is the previous cell's in the reference's loop order: (i,nj-1)
-// for the north edge, (i-1,nj) for the south edge.
-__device__ void final_topbottom(const ClsGeo& G, const double* vof, const double* phi, int i, int j, double& nx,
-                                double& ny) {
-    const PhiView p{G, phi};
+// The inner cell whose normal a cell that is not on the west or east edge
+// starts from: its own, or on the south and north edges (1 < i < ni) that of
+// the previous cell in the reference's loop order, (i,nj-1) for the north edge
+// and for the south edge (i-1,nj), which takes its own from (i-1,nj-1).
+__device__ __forceinline__ void normal_base(const ClsGeo& G, int i, int j, int& bi, int& bj) {
+    bi = j == 1 ? i - 1 : i;
+    bj = j == 1 || j == G.nj ? G.nj - 1 : j;
+    // within the grid's inner cells also where the caller will not use it
+    bi = min(max(bi, 2), G.ni - 1);
+}
+
+// final normal of interface cell (i,j) away from the west and east edges; p, vsb
+// the stencil and vofS of its base cell
+__device__ __forceinline__ void final_inner(const ClsGeo& G, const double* vof, const double* phi, const Stencil& p,
+                                            double vsb, int i, int j, double& nx, double& ny) {
     const int ni = G.ni, nj = G.nj;
-    if (!cls_of(G, vof, i, j)) {
-        nx = 0.0;
-        ny = 1.0;
-        return;
+    int bi, bj;
+    normal_base(G, i, j, bi, bj);
+    const bool edge = j == 1 || j == nj;
+    bool own = true;  // the base cell's normal is wanted
+    if (j == nj) own = cls_of(G, vof, i, nj - 1) != 0;
+    if (j == 1) own = i > 2 && cls_of(G, vof, i - 1, nj) && cls_of(G, vof, i - 1, nj - 1);
+    nx = 0.0;
+    ny = 1.0;
+    if (own) {
+        normal_irre(G, p, vsb, bi, bj, nx, ny);
+        normalise(nx, ny);
     }
-    double snx, t;
-    if (j == nj) {
-        final_interior(G, vof, phi, i, nj - 1, snx, t);
-    } else {  // j == 1: previous cell is (i-1, nj)
-        const int ip = i - 1;
-        if (ip == 1) {
-            final_side(G, vof, phi, 1, nj, snx, t);
-        } else if (cls_of(G, vof, ip, nj)) {
-            double a, b;
-            final_interior(G, vof, phi, ip, nj - 1, a, b);
-            b = edge_ny(p, ip, nj, nj);
-            normalise(a, b);
-            snx = a;
+    if (!edge) return;
+    const PhiView q{G, phi};
+    if (j == 1) {
+        if (i == 2) {
+            double t;
+            final_side(G, vof, phi, 1, nj, nx, t);
+        } else if (cls_of(G, vof, i - 1, nj)) {
+            double b = edge_ny(q, i - 1, nj, nj);
+            normalise(nx, b);
         } else {
-            snx = 0.0;
+            nx = 0.0;
         }
     }
-    nx = snx;
-    ny = edge_ny(p, i, j, nj);
+    ny = edge_ny(q, i, j, nj);
     normalise(nx, ny);
 }
 
@@ -744,24 +777,31 @@ struct ReconOut {
     double* fl;
 };
 
+// what the PLIC face fluxes of a cell need besides its plane
+struct FluxIn {
+    double nxs, nys, phis, w, w0;
+};
+
 // the PLIC face fluxes of cell c (VOFEPS < vof < 1-VOFEPS) with its plane: the
 // far-face flux where the cell is upwind of its far face, the near-face flux
 // where it is upwind of its near face -- exactly the values vof_flux would
-// compute for them in the sweep
+// compute for them in the sweep (a loop over the two keeps one copy of the code)
 template <bool X>
-__device__ __forceinline__ void cell_fluxes(const ClsGeo& G, int c, double f, double nx, double ny, double d,
-                                            double dtv, double* __restrict__ fr, double* __restrict__ fl) {
+__device__ __forceinline__ void cell_fluxes(const FluxIn& F, int c, double f, double vs, double nx, double ny, double d,
+                                            double hx, double hy, double dtv, double* __restrict__ fr,
+                                            double* __restrict__ fl) {
     if (f >= (1.0 - VOFEPS) || f <= VOFEPS) return;  // not vof_flux's PLIC branch
-    const int i = c % G.ni + 1, j = c / G.ni + 1;
-    const Line<X> L{G, X ? j : i};
-    const int a = X ? i : j;
-    const double hx = G.dx[i - 1], hy = G.dy[j - 1];
-    const double nxs = G.nxS[c], nys = G.nyS[c], phis = G.phiS[c], vs = G.vofS[c];
-    const double w = L.vel(a), w0 = L.vel(a - 1);
-    if (X ? (w >= 0.0) : (w > 0.0))
-        fr[c] = plic_face_flux<X>(1, nx, ny, d, f, nxs, nys, phis, vs, hx, hy, w * dtv);
-    if (!(X ? (w0 >= 0.0) : (w0 > 0.0)))
-        fl[c] = -plic_face_flux<X>(-1, nx, ny, d, f, nxs, nys, phis, vs, hx, hy, -w0 * dtv);
+#pragma unroll 1
+    for (int side = 1; side >= -1; side -= 2) {
+        const double w = side > 0 ? F.w : F.w0;
+        if ((X ? (w >= 0.0) : (w > 0.0)) != (side > 0)) continue;
+        const double flux = plic_face_flux<X>(side, nx, ny, d, f, F.nxs, F.nys, F.phis, vs, hx, hy,
+                                              side > 0 ? w * dtv : -w * dtv);
+        if (side > 0)
+            fr[c] = flux;
+        else
+            fl[c] = -flux;
+    }
 }
 
 // Interface_Reconstruct of cell c: its normal and plane constant where it is an
@@ -776,24 +816,38 @@ template <int DIR>
 __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __restrict__ vof,
                                            const double* __restrict__ phi, const ReconOut& O, double dtv, int c,
                                            bool full) {
-    const double vf = vof[c];
-    double nx = 0.0, ny = 1.0, d = 0.0;
     int i = c % G.ni + 1, j = c / G.ni + 1;
+    double vf = 0.0, vsc = 0.0, hxc = 0.0, hyc = 0.0;
+    FluxIn F{};
+    double nx = 0.0, ny = 1.0, d = 0.0;
     bool own = true, itf = false;
     for (;;) {
+        // everything a two-phase cell may need in one trip to memory
         const size_t p = cix(G, i, j);
-        const double v = vof[p], vs = G.vofS[p];
-        const int cl = recon_class(v, vs);
+        int bi, bj;
+        normal_base(G, i, j, bi, bj);
+        const double v = vof[p], vs = G.vofS[p], vsb = G.vofS[cix(G, bi, bj)];
         const double hx = G.dx[i - 1], hy = G.dy[j - 1];
+        const Stencil S = stencil(G, phi, bi, bj);
+        if (own) {
+            vf = v;
+            vsc = vs;
+            hxc = hx;
+            hyc = hy;
+            if (DIR != FLUX_NONE) {
+                const Line<DIR == FLUX_X> L{G, DIR == FLUX_X ? j : i};
+                const int a = DIR == FLUX_X ? i : j;
+                F = FluxIn{G.nxS[p], G.nyS[p], G.phiS[p], L.vel(a), L.vel(a - 1)};
+            }
+        }
+        const int cl = recon_class(v, vs);
         bool set = true;
         if (cl) {
             double mx, my;
-            if (i > 1 && i < G.ni && j > 1 && j < G.nj)
-                final_interior(G, vof, phi, i, j, mx, my);
-            else if (i == 1 || i == G.ni)
+            if (i == 1 || i == G.ni)
                 final_side(G, vof, phi, i, j, mx, my);
             else
-                final_topbottom(G, vof, phi, i, j, mx, my);
+                final_inner(G, vof, phi, S, vsb, i, j, mx, my);
             if (cl == 1)
                 d = plic_distance(v, mx, my, hx, hy);
             else
@@ -823,7 +877,8 @@ __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __rest
         O.P.ny[c] = ny;
     }
     if (itf) O.P.dis[c] = d;
-    if (DIR != FLUX_NONE) cell_fluxes<DIR == FLUX_X>(G, c, vf, nx, ny, d, dtv, O.fr, O.fl);
+    if (DIR != FLUX_NONE)
+        cell_fluxes<DIR == FLUX_X>(F, c, vf, vsc, nx, ny, d, hxc, hyc, dtv, O.fr, O.fl);
 }
 
 // Interface_Reconstruct over the grid: a workgroup lists the cells of its 64 x
@@ -838,8 +893,10 @@ __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __rest
 // Bound by the latency of one cell's chain of divisions and square roots, with
 // SCAN also by 16 bytes a cell.  As a scan, a kernel over the listed cells, one
 // over those with a stale plane constant and one for the fluxes it took 19.6 us
-// at 333 x 171 and 37.3 us at 2048^2; in one, scanning, 16.6 and 34 us; with the
-// bits of the sweep before it 10.9 and 13.9 us (17.1 us listing the sources).
+// at 333 x 171 and 37.3 us at 2048^2; in one with the bits of the sweep before it
+// 10.9 and 13.9 us; with a cell's operands in one trip to memory and one copy of
+// the normal's and the flux's code (80 to 51 KB) 9.4 and 12.7 us (16.3 us listing
+// the sources; scanning 15.1 and 30.8 us).
 constexpr int RECON_NT = 256;
 constexpr int RECON_H = 64;  // rows per workgroup: one a lane when the words are listed
 template <int DIR, bool SCAN>
