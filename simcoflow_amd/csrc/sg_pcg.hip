@@ -51,6 +51,12 @@ __device__ inline bool reliable_due(const PcgScalars* sc) {
     return sc->active && sc->rr < RELIABLE_DROP * sc->rr_ref;
 }
 
+// the direction's beta from s = (r,z), (z_new,q_old)
+__device__ __forceinline__ double rz_beta(const PcgScalars* sc, const double (&s)[2]) {
+    if (sc->first) return 0.0;
+    return sc->flexible ? -sc->alpha * s[1] / sc->rz_old : s[0] / sc->rz_old;
+}
+
 // one reduction slot: NRED planes of per-block partials
 struct Slots {
     double* part;
@@ -128,17 +134,36 @@ __global__ void __launch_bounds__(256) k_dot_mu(Dims D, const double* __restrict
 // perturbed system, which the FP64 residual recomputation then has to undo
 // at a rate set by the condition number), the stencil sums and (p,q) in
 // FP64.
+// The scalars a kernel reads come from a finalize launch before it, or, with
+// nsum > 0, the kernel works them out itself: every block adds the nsum partials
+// up (the same sums in every bit), block 0 records the results, and no field it
+// writes is read by another block.  On a small grid a finalize is a launch and a
+// trip to memory between two kernels of about its own length: two finalizes
+// fewer an iteration take a 128 x 256 solve of 34 iterations from 3.71 to 3.54 ms.
 constexpr int DW = 64, DH = 16;
 template <typename V>
 __global__ void __launch_bounds__(256) k_dir_apply(Dims D, const double* __restrict__ diag,
                                                    const double* __restrict__ cE, const double* __restrict__ cN,
                                                    const V* __restrict__ z, const V* __restrict__ pold,
                                                    const double* __restrict__ w, V* __restrict__ pnew,
-                                                   V* __restrict__ q, Slots S, const PcgScalars* sc) {
+                                                   V* __restrict__ q, Slots S, PcgScalars* sc, Slots Srz, int nsum) {
     if (!sc->active) return;
     constexpr int RW = DW + 2, RH = DH + 2;
     __shared__ V sp[RH][RW];
-    const V beta = (V)sc->beta;
+    double beta_d;
+    if (nsum > 0) {
+        double sum[2];
+        sum_all<2>(Srz.part, Srz.max_blocks, nsum, sum);
+        beta_d = rz_beta(sc, sum);
+        if (threadIdx.x == 0 && blockIdx.x + blockIdx.y == 0) {
+            sc->rz = sum[0];
+            sc->zq = sum[1];
+            sc->beta = beta_d;
+        }
+    } else {
+        beta_d = sc->beta;
+    }
+    const V beta = (V)beta_d;
     const V mu = w ? (V)sc->mu_eff : V(0);
     // the first direction reads no old one: p_old still holds the last
     // solve's, which may not be finite after a failed solve (0 * NaN)
@@ -187,12 +212,24 @@ template <typename V>
 __global__ void __launch_bounds__(256) k_update(Dims D, const V* __restrict__ p, const V* __restrict__ q,
                                                 const double* __restrict__ w, const double* __restrict__ aw,
                                                 double* __restrict__ x, V* __restrict__ r, Slots S,
-                                                const PcgScalars* sc) {
+                                                PcgScalars* sc, Slots Spq, int nsum) {
     if (!sc->active) return;
-    const double alpha = sc->alpha;
-    const V alv = (V)alpha;
     const int i = blockIdx.x * TX + threadIdx.x;
     const int j = blockIdx.y * TY + threadIdx.y;
+    double alpha;
+    if (nsum > 0) {
+        double sum[1];
+        sum_all<1>(Spq.part, Spq.max_blocks, nsum, sum);
+        alpha = sc->rz / sum[0];
+        if (threadIdx.x + threadIdx.y == 0 && blockIdx.x + blockIdx.y == 0) {
+            sc->pq = sum[0];
+            sc->alpha = alpha;
+            sc->first = 0;
+        }
+    } else {
+        alpha = sc->alpha;
+    }
+    const V alv = (V)alpha;
     double v[1] = {0.0};
     if (i < D.ni && j < D.nj) {
         const size_t k = D.off(i, j);
@@ -285,8 +322,7 @@ __global__ void __launch_bounds__(NTF) k_finalize(Slots S, int nblocks, int mode
         finalize_sum<2, NTF>(S.part, S.max_blocks, nblocks, s);
         if (threadIdx.x != 0) return;
         if (mode == FIN_RZ) {
-            double beta = 0.0;
-            if (!sc->first) beta = sc->flexible ? -sc->alpha * s[1] / sc->rz_old : s[0] / sc->rz_old;
+            const double beta = rz_beta(sc, s);
             sc->rz = s[0];
             sc->zq = s[1];
             sc->beta = beta;
@@ -354,6 +390,14 @@ Slots slots(Ctx* c, int s) {
 bool learned(Ctx* c) { return (c->prm.warm_start == 2 || c->prm.warm_start == 3) && (c->nn.on || c->nn.ext_on); }
 bool deflating(Ctx* c) { return learned(c) && c->nn.deflate; }
 
+// up to how many partials their consumers add up themselves: one load a thread.
+// Solves with and without (ms, FP64): 64 x 128 1.73 / 1.82, 256^2 3.61 / 3.78,
+// 384^2 7.20 / 7.55, 512^2 (256 partials) 3.59 / 3.73.  With four loads a thread,
+// up to 1024 partials, 1024^2 lost 1.91 -> 2.11 (mixed): there every block of a grid
+// that fills the chip waits for sums that one block makes while others work.
+constexpr int FUSE_MAX = SUM_MAX;
+static_assert(FUSE_MAX <= SUM_MAX && SUM_MAX <= NTF, "the sums must be those of a finalize launch");
+
 // one PCG iteration (V-cycle + direction + update), enqueued on the stream;
 // V = the vector precision, A the operator of that precision
 template <typename V>
@@ -376,22 +420,28 @@ int enqueue_iteration_t(Ctx* c, int parity, V* r, V* z, V* q, V* p0, V* p1) {
                            (const PcgScalars*)c->sc);
         nb_rz = nb;
     }
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S1, nb_rz, (int)FIN_RZ, c->sc, 0.0);
+    const dim3 gd((c->ni + DW - 1) / DW, (c->nj + DH - 1) / DH);
+    const int nb_pq = (int)(gd.x * gd.y);
+    // without a deflation vector between them, the kernels that use (r,z) and
+    // (p,q) add the partials up themselves where those are few enough
+    const bool defl = deflating(c);
+    const int sum_rz = !defl && nb_rz <= FUSE_MAX ? nb_rz : 0, sum_pq = !defl && nb_pq <= FUSE_MAX ? nb_pq : 0;
+    if (!sum_rz) hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S1, nb_rz, (int)FIN_RZ, c->sc, 0.0);
     const double* w = nullptr;
-    if (deflating(c)) {
+    if (defl) {
         Slots S6 = slots(c, 6);
         hipLaunchKernelGGL(k_dot_mu<V>, g, b, 0, s, D, (const double*)c->nn.aw, (const V*)z, S6,
                            (const PcgScalars*)c->sc);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S6, nb, (int)FIN_MU, c->sc, 0.0);
         w = c->nn.w;
     }
-    const dim3 gd((c->ni + DW - 1) / DW, (c->nj + DH - 1) / DH);
     hipLaunchKernelGGL(k_dir_apply<V>, gd, dim3(256), 0, s, D, (const double*)A.diag, (const double*)A.cE,
-                       (const double*)A.cN, (const V*)z, (const V*)pold, w, pnew, q, S2, (const PcgScalars*)c->sc);
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S2, (int)(gd.x * gd.y), (int)(w ? FIN_PQ_DEFL : FIN_PQ),
-                       c->sc, 0.0);
+                       (const double*)A.cN, (const V*)z, (const V*)pold, w, pnew, q, S2, c->sc, S1, sum_rz);
+    if (!sum_pq)
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S2, nb_pq, (int)(w ? FIN_PQ_DEFL : FIN_PQ), c->sc,
+                           0.0);
     hipLaunchKernelGGL(k_update<V>, g, b, 0, s, D, (const V*)pnew, (const V*)q, w, w ? (const double*)c->nn.aw : nullptr,
-                       c->x, r, S3, (const PcgScalars*)c->sc);
+                       c->x, r, S3, c->sc, S2, sum_pq);
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S3, nb, (int)FIN_RR, c->sc, 0.0);
     if (sizeof(V) == 4 && parity == 1) {
         // FP32 vectors: recompute r from x in FP64 when it is due, keeping

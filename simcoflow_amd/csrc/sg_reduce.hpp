@@ -70,4 +70,34 @@ __device__ inline void finalize_sum(const double* partials, int max_blocks, int 
     block_reduce<NV, NT>(s);
 }
 
+// finalize_sum of a kernel of at least SUM_MAX threads, for every thread of a
+// block of 256: the same sums in every bit (the butterflies of the same groups
+// of 64 partials, their results added in the same order), so a kernel can use
+// them without a finalize launch before it.  nblocks <= SUM_MAX.
+constexpr int SUM_MAX = 256;
+template <int NV>
+__device__ __forceinline__ void sum_all(const double* __restrict__ partials, int max_blocks, int nblocks,
+                                        double (&s)[NV]) {
+    __shared__ double lds[SUM_MAX / 64][NV];
+    const int tid = threadIdx.x + threadIdx.y * blockDim.x;
+    if ((tid & ~63) < nblocks) {
+        double v[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = tid < nblocks ? 0.0 + partials[(size_t)k * max_blocks + tid] : 0.0;
+        wave_reduce<NV>(v);
+        if ((tid & 63) == 0) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) lds[tid >> 6][k] = v[k];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        s[k] = 0.0;
+#pragma unroll
+        for (int g = 0; g < SUM_MAX / 64; ++g)
+            if (g * 64 < nblocks) s[k] += lds[g][k];
+    }
+}
+
 }  // namespace sg
