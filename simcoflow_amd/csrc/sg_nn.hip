@@ -29,14 +29,50 @@ __device__ __forceinline__ floatx4 mfma(const bf16x8& a, const bf16x8& b, const 
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// The results of MB x NPB tiles of channels c0.. and pixels x0.. of one row: a
+// lane holds D[co = mb*16 + 4*q4 + r][px = x0 + q*16 + r16], r = 0..3.  Applies
+// ReLU (optionally after adding a skip tensor), masks by aux > 0 (data gradient
+// through a ReLU), writes plain, or writes channel 0 as FP32 (the output layer).
+template <int MB, int NPB>
+__device__ __forceinline__ void conv_store(const floatx4 (&acc)[MB][NPB], const T4& in, const T4& out, const T4& aux,
+                                           float* __restrict__ yo, int epi, int c0, int b, int y, int x0) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
+#pragma unroll
+    for (int q = 0; q < NPB; ++q) {
+        const int px = x0 + q * 16 + r16;
+        if (epi == E_OUT) {
+            if (q4 == 0) yo[((size_t)b * in.H + y) * in.W + px] = acc[0][q][0];
+            continue;
+        }
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) {
+            const int co = c0 + mb * 16 + 4 * q4;
+            float v[4] = {acc[mb][q][0], acc[mb][q][1], acc[mb][q][2], acc[mb][q][3]};
+            if (epi == E_RELU_SKIP || epi == E_MASK) {
+                const bf16x4 a = *(const bf16x4*)(aux.p + t4off(aux, b, y + 1, px + 1) + co);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float av = (float)a[r];
+                    v[r] = epi == E_MASK ? (av > 0.f ? v[r] : 0.f) : v[r] + av;
+                }
+            }
+            if (epi == E_RELU || epi == E_RELU_SKIP) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
+            }
+            bf16x4 o;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = (bf16)v[r];
+            *(bf16x4*)(out.p + t4off(out, b, y + 1, px + 1) + co) = o;
+        }
+    }
+}
+
 // out(b,y,x,co) = sum_{tap,ci} wt[co][tap*CIN+ci] * in(b, y+dy-1, x+dx-1, ci)
 // One wave: 16*NPB pixels of one row and COUT/CG of the output channels
 // (CG > 1 on small levels, where one wave per pixel group would leave most
 // of the chip idle; each output still sums over (tap, ci) in the same
-// order).  The epilogue
-// applies ReLU (optionally after adding a skip tensor), masks by aux > 0
-// (data gradient through a ReLU), writes plain, or writes channel 0 as FP32
-// (the output layer).
+// order).
 template <int CIN, int COUT, int NPB, int CG>
 __global__ void __launch_bounds__(256) k_conv(T4 in, const bf16* __restrict__ wt, T4 out, T4 aux,
                                               float* __restrict__ yo, int nb, int epi) {
@@ -82,35 +118,114 @@ __global__ void __launch_bounds__(256) k_conv(T4 in, const bf16* __restrict__ wt
             for (int q = 0; q < NPB; ++q) acc[mb][q] = mfma(av, bv[q], acc[mb][q]);
         }
     }
-    // lane holds D[co = mb*16 + 4*q4 + r][px = x0 + q*16 + r16], r = 0..3
+    conv_store<MB, NPB>(acc, in, out, aux, yo, epi, g * MB * 16, b, y, x0);
+}
+
+// k_conv for many pixels: a wave takes a strip of 16 NPB pixels by `rows` rows,
+// and 16 MB channels.  A row of the input is loaded once and multiplied into
+// the three output rows it belongs to, so a strip loads rows + 2 rows where
+// k_conv loads 3 rows' worth for each; the weights of the workgroup's channels
+// stand in LDS in the order the MFMA takes them (one 16-byte read a lane, no
+// conflicts), where k_conv reads them again from the caches for every row.
+// Chunks of the reduction do not run over the end of a tap row: 3 x 8 channels
+// fill 24 of 32, 3 x 16 take two chunks.
+//
+// At 16 images, us a layer against k_conv: 16 x 16 at 256^2 24.4 / 26.4, 32 x 16
+// 30.6 / 41.2, 32 x 32 at 128^2 18.3 / 21.5, 64 x 32 40.9 / 37.2 forward with the
+// skip, 64 x 64 at 64^2 22.8 / 28.5, 128 x 64 40.0 / 51.9, 128 x 128 at 32^2 30.3 /
+// 43.0.  The narrow layers are bound by their activations' bytes (2.7 TB/s at 24.4
+// us), the wide ones by the loads' latency at two waves a SIMD.
+template <int CIN>
+struct StripK {
+    static constexpr int FR = CIN == 8 ? 1 : CIN == 16 ? 2 : 3 * CIN / 32;  // chunks of a tap row
+    // column tap (3: none) and first channel of a lane's 8 in chunk f
+    __host__ __device__ static constexpr int dx(int f, int q4) {
+        return CIN == 8 ? q4 : CIN == 16 ? (f == 0 ? q4 >> 1 : (q4 < 2 ? 2 : 3)) : f / (CIN >= 32 ? CIN / 32 : 1);
+    }
+    __host__ __device__ static constexpr int ci(int f, int q4) {
+        return CIN == 8 ? 0 : CIN == 16 ? 8 * (q4 & 1) : f % (CIN >= 32 ? CIN / 32 : 1) * 32 + 8 * q4;
+    }
+};
+template <int CIN, int COUT, int MB, int NPB>
+__global__ void __launch_bounds__(256, 2) k_conv_strip(T4 in, const bf16* __restrict__ wt, T4 out, T4 aux,
+                                                    float* __restrict__ yo, int nb, int epi, int rows) {
+    using K = StripK<CIN>;
+    constexpr int FR = K::FR, KP = kpad(CIN), CG = COUT / 16 / MB;
+    constexpr bool AHEAD = FR * NPB <= 12;  // the next row's loads in flight
+    static_assert(COUT % (16 * MB) == 0, "channel groups must split the 16-channel blocks");
+    __shared__ bf16x8 ws[3 * FR * MB * 64];
+    const int lane = threadIdx.x & 63, r16 = lane & 15, q4 = lane >> 4;
+    const int g = (int)(blockIdx.x % CG);
+    const bf16x8 zero = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
+    for (int e = threadIdx.x; e < 3 * FR * MB * 64; e += 256) {
+        const int l = e & 63, f = e >> 6, mb = f % MB, fr = f / MB % FR, dy = f / MB / FR;
+        const int dx = K::dx(fr, l >> 4), ci = K::ci(fr, l >> 4);
+        const int co = (g * MB + mb) * 16 + (l & 15);
+        ws[e] = dx < 3 ? *(const bf16x8*)(wt + (size_t)co * KP + (dy * 3 + dx) * CIN + ci) : zero;
+    }
+    __syncthreads();
+    const int tiles = in.W / (16 * NPB), segs = (in.H + rows - 1) / rows;
+    const long strip = (long)(blockIdx.x / CG) * 4 + (threadIdx.x >> 6);
+    if (strip >= (long)nb * segs * tiles) return;
+    const int x0 = (int)(strip % tiles) * (16 * NPB);
+    const long t = strip / tiles;
+    const int y0 = (int)(t % segs) * rows, b = (int)(t / segs);
+    const int n = min(rows, in.H - y0);
+    const bf16* src = in.p + t4off(in, b, y0, x0 + r16);
+    const long step = (long)(in.W + 2) * CIN;
+    auto load = [&](int iy, bf16x8 (&v)[FR][NPB]) {
 #pragma unroll
-    for (int q = 0; q < NPB; ++q) {
-        const int px = x0 + q * 16 + r16;
-        if (epi == E_OUT) {
-            if (q4 == 0) yo[((size_t)b * in.H + y) * in.W + px] = acc[0][q][0];
-            continue;
+        for (int f = 0; f < FR; ++f) {
+            const int dx = K::dx(f, q4);
+            const bf16* p = src + iy * step + (dx < 3 ? dx * CIN : 0) + K::ci(f, q4);
+#pragma unroll
+            for (int q = 0; q < NPB; ++q) v[f][q] = CIN >= 32 || dx < 3 ? *(const bf16x8*)(p + q * 16 * CIN) : zero;
         }
+    };
+    typedef floatx4 Acc[MB][NPB];
+    auto clear = [&](Acc& a) {
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            const int co = (g * MB + mb) * 16 + 4 * q4;
-            float v[4] = {acc[mb][q][0], acc[mb][q][1], acc[mb][q][2], acc[mb][q][3]};
-            if (epi == E_RELU_SKIP || epi == E_MASK) {
-                const bf16x4 a = *(const bf16x4*)(aux.p + t4off(aux, b, y + 1, px + 1) + co);
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float av = (float)a[r];
-                    v[r] = epi == E_MASK ? (av > 0.f ? v[r] : 0.f) : v[r] + av;
-                }
+            for (int q = 0; q < NPB; ++q) a[mb][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto add = [&](int dy, const bf16x8 (&v)[FR][NPB], Acc& a) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                const bf16x8 av = ws[((dy * FR + f) * MB + mb) * 64 + lane];
+#pragma unroll
+                for (int q = 0; q < NPB; ++q) a[mb][q] = mfma(av, v[f][q], a[mb][q]);
             }
-            if (epi == E_RELU || epi == E_RELU_SKIP) {
+    };
+    Acc acc[3];
+    bf16x8 cur[FR][NPB], nxt[AHEAD ? FR : 1][AHEAD ? NPB : 1];
+    // input row iy of the strip: tap row 0 of output row iy, 1 of iy - 1, 2 of iy - 2
+    auto row = [&](int iy, Acc& a, Acc& m, Acc& z) {
+        if (iy > n + 1) return;
+        if constexpr (AHEAD) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = v[r] > 0.f ? v[r] : 0.f;
-            }
-            bf16x4 o;
+            for (int f = 0; f < FR; ++f)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) o[r] = (bf16)v[r];
-            *(bf16x4*)(out.p + t4off(out, b, y + 1, px + 1) + co) = o;
+                for (int q = 0; q < NPB; ++q) cur[f][q] = nxt[f][q];
+            if (iy <= n) load(iy + 1, nxt);
+        } else {
+            load(iy, cur);
         }
+        if (iy >= 2) add(2, cur, z);
+        if (iy >= 1 && iy <= n) add(1, cur, m);
+        if (iy >= 2) conv_store<MB, NPB>(z, in, out, aux, yo, epi, g * MB * 16, b, y0 + iy - 2, x0);
+        if (iy < n) {
+            clear(a);
+            add(0, cur, a);
+        }
+    };
+    if constexpr (AHEAD) load(0, nxt);
+    for (int iy = 0; iy < n + 2; iy += 3) {
+        row(iy, acc[0], acc[2], acc[1]);
+        row(iy + 1, acc[1], acc[0], acc[2]);
+        row(iy + 2, acc[2], acc[1], acc[0]);
     }
 }
 
@@ -368,20 +483,25 @@ __global__ void __launch_bounds__(256) k_poolT_add_mask(T4 dd, T4 skip, T4 act, 
     *(bf16x8*)(P.p + t4off(P, b, y + 1, x + 1) + c8) = o;
 }
 
-// loss = sum mask*(y-t)^2 / n ; gout channel 0 = 2 mask (y-t) / n
+// loss = sum mask*(y-t)^2 / n ; gout channel 0 = 2 mask (y-t) / n.  A workgroup
+// takes LOSS_PX pixels: bound by the adds to the one sum, one a workgroup (256
+// pixels each: 57.6 us at 16 x 256 x 256 pixels; 2048: 22.7).
+constexpr int LOSS_PX = 2048;
 __global__ void __launch_bounds__(256) k_loss(const float* __restrict__ y, const float* __restrict__ t,
                                               const float* __restrict__ m, T4 g, int nb, float inv_n,
                                               float* __restrict__ loss) {
     __shared__ float red[4];
     const long n = (long)nb * g.H * g.W;
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
     float l = 0.f;
-    if (e < n) {
+#pragma unroll
+    for (int k = 0; k < LOSS_PX / 256; ++k) {
+        const long e = (long)blockIdx.x * LOSS_PX + k * 256 + threadIdx.x;
+        if (e >= n) break;
         const int x = (int)(e % g.W);
         const long r = e / g.W;
         const int yy = (int)(r % g.H), b = (int)(r / g.H);
         const float d = m[e] > 0.f ? y[e] - t[e] : 0.f;
-        l = d * d * inv_n;
+        l += d * d * inv_n;
         g.p[t4off(g, b, yy + 1, x + 1)] = (bf16)(2.f * d * inv_n);
     }
     for (int o = 32; o >= 1; o >>= 1) l += __shfl_xor(l, o, 64);
@@ -453,8 +573,35 @@ void conv_split(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb,
         conv_launch<CIN, COUT, NPB, 1>(n, in, w, out, aux, yo, nb, epi, waves);
 }
 
+// Strips of as many rows as leave STRIP_WAVES waves, two a SIMD: with 4096 and
+// 8192 a 16 x 16 layer of 16 x 256 x 256 pixels takes 26.5 and 28.1 us against
+// 24.4, a 32 x 32 one of 16 x 128 x 128 22.7 and 22.7 against 18.3.  64-pixel
+// strips where those can be two rows high; else, for the layers whose work per
+// pixel is large, 32-pixel ones (64 x 64 at 16 x 64 x 64: 22.8 against 27.6 us),
+// one row high if need be (128 x 128 at 16 x 32 x 32: 30.3 against k_conv's 43.0).
+// With fewer tiles k_conv, which splits the channels further, keeps the chip fuller.
+constexpr long STRIP_WAVES = 2048;
+
+template <int CIN, int COUT, int MB, int NPB>
+bool conv_strip(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb, int epi, long least) {
+    constexpr int CG = COUT / 16 / MB;
+    const long tiles = in.W / (16 * NPB), all = nb * in.H * tiles * CG;
+    if (in.W % (16 * NPB) || all < least) return false;
+    const int rows = (int)std::min(16l, all / STRIP_WAVES);
+    const long strips = nb * ((in.H + rows - 1) / rows) * tiles;
+    hipLaunchKernelGGL((k_conv_strip<CIN, COUT, MB, NPB>), dim3((unsigned)((strips + 3) / 4 * CG)), dim3(256), 0,
+                       n->stream, in, w, out, aux, yo, nb, epi, rows);
+    return true;
+}
+
 template <int CIN, int COUT>
 int conv(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb, int epi) {
+    constexpr int MB = COUT == 16 ? 1 : 2;
+    if ((CIN < 128 && conv_strip<CIN, COUT, MB, (CIN < 128 ? 4 : 2)>(n, in, w, out, aux, yo, nb, epi, 2 * STRIP_WAVES)) ||
+        ((CIN >= 64 || in.W % 64) && conv_strip<CIN, COUT, MB, 2>(n, in, w, out, aux, yo, nb, epi, STRIP_WAVES))) {
+        SG_HIP(hipGetLastError());
+        return SG_OK;
+    }
     // four 16-pixel groups per wave where that still leaves ~4 waves per CU
     if (in.W % 64 == 0 && (long)nb * in.H * (in.W / 64) >= 1024)
         conv_split<CIN, COUT, 4>(n, in, w, out, aux, yo, nb, epi, (long)nb * in.H * (in.W / 64));
@@ -656,7 +803,7 @@ int backward(Net* n, const bf16* Xp, const float* t, const float* mask, int nb) 
     hipLaunchKernelGGL(k_fill, dim3(blocks((long)n->nw)), dim3(256), 0, s, n->g, n->nw, 0.f);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, n->loss, (size_t)1, 0.f);
     const long npx = (long)nb * n->H * n->W;
-    hipLaunchKernelGGL(k_loss, dim3(blocks(npx)), dim3(256), 0, s, (const float*)n->y, t, mask, n->gout, nb,
+    hipLaunchKernelGGL(k_loss, dim3((unsigned)((npx + LOSS_PX - 1) / LOSS_PX)), dim3(256), 0, s, (const float*)n->y, t, mask, n->gout, nb,
                        1.f / (float)npx, n->loss);
     auto upT = [&](T4 d, T4 act, T4 P) {
         hipLaunchKernelGGL(k_upT_mask, dim3(blocks((long)nb * P.H * P.W * (P.C / 8))), dim3(256), 0, s, d, act, P,
