@@ -54,6 +54,7 @@ static void destroy(Ctx* c) {
     for (void* p : c->allocations) (void)hipFree(p);
     if (c->sc_host) (void)hipHostFree(c->sc_host);
     if (c->pred.sc_host) (void)hipHostFree(c->pred.sc_host);
+    if (c->part.flagged) (void)hipHostFree(c->part.flagged);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->ev2) (void)hipEventDestroy(c->ev2);

@@ -208,7 +208,7 @@ struct Net;
 struct ParticleState {
     int n = 0, cap = 0;
     double *x = nullptr, *y = nullptr, *u = nullptr, *v = nullptr, *d = nullptr;
-    unsigned* flagged = nullptr;
+    unsigned* flagged = nullptr;  // pinned: failed particles of each workgroup
     sg_particle_params last{};  // parameters and dt of the last tracking call
     double last_dt = 0.0;
     bool tracked = false;
