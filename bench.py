@@ -69,11 +69,10 @@ def log(msg):
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
-# The transport's sweep: 8 FP64 words per cell and sweep (16 per sweep pair:
-# read vof, phi, the two normal components, the plane constant, the face
-# velocity, the two apertures and vofS; write vof, phi and the normal and
-# plane constant the next reconstruction reads).
-SWEEP_WORDS = 8
+# The transport's sweep: 6 FP64 words per cell and sweep (first sweep: read vof,
+# phi and the face velocity, write vof, phi and temvf; second: read those and
+# temvf, write vof and phi; the solid's arrays only where there is solid).
+SWEEP_WORDS = 6
 
 # Algorithmic bytes per fine cell and PCG iteration (compulsory traffic at
 # the stored precision): operator apply 5 words (FP64 operator, the vector
@@ -571,7 +570,7 @@ def main():
     # roofline: the transport sweeps, the largest kernel family of the
     # metric's time step, timed launch by launch with HIP events during
     # steps of the metric's own path (a second pass, so the events stay out
-    # of the headline's timed steps); bytes: 8 FP64 words per cell per sweep
+    # of the headline's timed steps); bytes: SWEEP_WORDS FP64 words per cell
     log("transport sweeps timed with HIP events, metric path")
     lrn = (w, K) if w is not None else None
     ev = stepping(case, stags, 1, a.steps, a.warmup, learned=lrn, width=a.nn_width, previous=lrn is not None,
