@@ -221,8 +221,6 @@ int sg_ctx_create(int ni, int nj, const double* dx, const double* dy, const doub
         }
         CK(hipMemcpy(c->cls.xc, xc.data(), ni * sizeof(double), hipMemcpyHostToDevice));
         CK(hipMemcpy(c->cls.yc, yc.data(), nj * sizeof(double), hipMemcpyHostToDevice));
-        c->cls.xw = xc[0] - dx[0] / 2.0;
-        c->cls.dx0 = dx[0];
     }
     // cell-layout staging for the host-pointer test hooks (5 planes)
     c->stage = (double*)dev_alloc(c, 5 * ncell * sizeof(double));
@@ -747,7 +745,6 @@ int sg_set_centres(sg_ctx* ctx, const double* xc, const double* yc) {
     SG_HIP(hipMemcpyAsync(c->cls.xc, xc, c->ni * sizeof(double), hipMemcpyHostToDevice, c->stream));
     SG_HIP(hipMemcpyAsync(c->cls.yc, yc, c->nj * sizeof(double), hipMemcpyHostToDevice, c->stream));
     SG_HIP(hipStreamSynchronize(c->stream));
-    c->cls.xw = xc[0] - c->cls.dx0 / 2.0;
     return SG_OK;
 }
 
@@ -766,6 +763,8 @@ int sg_clsvof_advect_resident(sg_ctx* ctx, double dt, double time, const sg_clsv
         set_error("sg_clsvof_advect: dt must be >= 0");
         return SG_ERR_ARG;
     }
+    // the inflow level of X_Sweep (:1057-1059, depth, amp, kw and omega at the
+    // west edge) reaches ring cells only, which Boundary_Condition overwrites
     int rc = clsvof_advect(c, dt, p->nsub);
     if (rc) return rc;
     SG_HIP(hipGetLastError());

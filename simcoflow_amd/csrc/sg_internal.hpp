@@ -160,8 +160,6 @@ struct ClsBuffers {
     unsigned long long* bits = nullptr;  // the cells' class bits, four planes of mw x nj words
     unsigned char* open = nullptr;     // sweep tiles free of solid
     int mw = 0;                        // words per row
-    double xw = 0.0;                   // west edge x of the grid (host copy)
-    double dx0 = 0.0;                  // width of the first column (host copy)
 };
 
 // Staggered-cell geometry on the device: cell arrays first, then ghosted.
