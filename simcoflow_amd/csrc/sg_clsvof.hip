@@ -881,8 +881,8 @@ __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __rest
         cell_fluxes<DIR == FLUX_X>(F, c, vf, vsc, nx, ny, d, hxc, hyc, dtv, O.fr, O.fl);
 }
 
-// Interface_Reconstruct over the grid: a workgroup lists the cells of its 64 x
-// 64 that BIT_LIST names in LDS and works on them packed one per lane -- the
+// Interface_Reconstruct over the grid: a workgroup lists the cells of its 64 by
+// `rows` that BIT_LIST names in LDS and works on them packed one per lane -- the
 // geometry costs the same per cell wherever a cell lies, and packing keeps the
 // wavefronts of bulk liquid and gas out of it.  SCAN: the bits are not there
 // yet (a call's first reconstruction, or vofS has moved since the sweep), so
@@ -893,30 +893,42 @@ __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __rest
 // Bound by the latency of one cell's chain of divisions and square roots, with
 // SCAN also by 16 bytes a cell.  As a scan, a kernel over the listed cells, one
 // over those with a stale plane constant and one for the fluxes it took 19.6 us
-// at 333 x 171 and 37.3 us at 2048^2; in one with the bits of the sweep before it
-// 10.9 and 13.9 us; with a cell's operands in one trip to memory and one copy of
-// the normal's and the flux's code (80 to 51 KB) 9.4 and 12.7 us (16.3 us listing
-// the sources; scanning 15.1 and 30.8 us).
+// at 333 x 171 and 37.3 us at 2048^2; now 8.5 and 15.1 us (8.1 and 19.2 us listing
+// the sources, scanning 9.9 and 31.2).
+//
+// Few rows a workgroup keep a thread's share of a dense interface short, one
+// cell of 64 x 4; many keep the wavefronts full where it is sparse.  A call of six
+// sub-steps, us, by 4 / 8 / 16 / 32 rows (64 rows in front):
+//   bubbles on a lattice of 8 cells, 256^2             1465: 620 / 700 / 777 / 990
+//   the same at 512^2                                  2337: 1650 / 1665 / 1740 / 1910
+//   the same at 1024^2                                 5940: 5800 / 5715 / 5725 / 5757
+//   swarm 256^2                                         468: 334 / 357 / 356 / 400
+//   swarm 512^2                                         515: 434 / 428 / 441 / 438
+//   swarm 1024^2                                        795: - / 760 / 750 / 765
+//   swarm 1448^2                                       1120: - / 1190 / 1125 / 1115
+//   swarm 2048^2                                       1835: - / 2024 / 1893 / 1850
 constexpr int RECON_NT = 256;
-constexpr int RECON_H = 64;  // rows per workgroup: one a lane when the words are listed
+constexpr int RECON_H = 32;  // most rows of a workgroup (one a lane when the words are listed: 64 at most)
+int recon_rows(size_t cells) { return cells < (1ull << 18) ? 4 : cells < (1ull << 21) ? 16 : RECON_H; }
 template <int DIR, bool SCAN>
 __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __restrict__ vof,
                                                     const double* __restrict__ phi, ReconOut O, Bits B, double dtv,
-                                                    int full, int* __restrict__ srcs, unsigned* __restrict__ nsrc) {
+                                                    int rows, int full, int* __restrict__ srcs,
+                                                    unsigned* __restrict__ nsrc) {
     constexpr int NW = RECON_NT / 64, R = RECON_H / NW;
     __shared__ unsigned long long words[2][SCAN ? RECON_H : 1];
     __shared__ unsigned short list[64 * RECON_H];
     __shared__ unsigned gbase;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i0 = blockIdx.x * 64, jb = blockIdx.y * RECON_H;
+    const int i0 = blockIdx.x * 64, jb = blockIdx.y * rows;
     if (SCAN) {
         const int i = i0 + lane + 1;
         // every row's operands loaded before any test
         double vf[R], vs[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int j = jb + r * NW + w + 1;
-            const bool in = i <= G.ni && j <= G.nj;
+            const int row = r * NW + w, j = jb + row + 1;
+            const bool in = row < rows && i <= G.ni && j <= G.nj;
             const size_t c = in ? cix(G, i, j) : 0;
             vf[r] = in ? vof[c] : 0.0;
             vs[r] = in ? G.vofS[c] : 0.0;
@@ -924,7 +936,7 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int row = r * NW + w, j = jb + row + 1;
-            const bool in = i <= G.ni && j <= G.nj;
+            const bool row_in = row < rows && j <= G.nj, in = row_in && i <= G.ni;
             unsigned long long b[NBITS];
             b[BIT_LIST] = __ballot(in && bit_list(vf[r], vs[r]));
             b[BIT_SRC] = __ballot(in && bit_src(vf[r], vs[r]));
@@ -934,7 +946,7 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
                 words[0][row] = b[BIT_LIST];
                 words[1][row] = b[BIT_SRC];
             }
-            if (lane < NBITS && j <= G.nj) {
+            if (lane < NBITS && row_in) {
                 const unsigned long long v = lane == 0 ? b[0] : lane == 1 ? b[1] : lane == 2 ? b[2] : b[3];
                 B.w[lane][(size_t)(j - 1) * B.mw + blockIdx.x] = v;
             }
@@ -942,19 +954,22 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
         __syncthreads();
     }
     // one row's word a lane, in every wavefront
-    const bool row_in = jb + lane < G.nj;
     unsigned long long wl = 0ull, ws = 0ull;
-    if (SCAN) {
-        wl = words[0][lane];
-        if (srcs) ws = words[1][lane];
-    } else if (row_in) {
+    if (lane < rows && jb + lane < G.nj) {
         const size_t at = (size_t)(jb + lane) * B.mw + blockIdx.x;
-        wl = B.w[BIT_LIST][at];
-        if (srcs) ws = B.w[BIT_SRC][at];
+        wl = SCAN ? words[0][lane] : B.w[BIT_LIST][at];
+        if (srcs) ws = SCAN ? words[1][lane] : B.w[BIT_SRC][at];
     }
-    // where each row's cells start in the two lists: an inclusive scan of the
-    // packed counts (low and high 16 bits, at most 4096 of each) over the rows
-    const unsigned own = (unsigned)__popcll(wl) | ((unsigned)__popcll(ws) << 16);
+    // the cells on the west and east edges, whose normals take a walk along a run
+    // of them, come first in the list, a lane each: no thread has two walks to do
+    // (256^2, an interface cell everywhere: 141 us against 2940 with up to sixteen)
+    const int ei = G.ni - 1 - i0;
+    const unsigned long long west = i0 == 0 ? 1ull : 0ull, east = ei < 64 ? 1ull << ei : 0ull;
+    const unsigned long long wrows = __ballot((wl & west) != 0ull), erows = __ballot((wl & east) != 0ull);
+    const unsigned nw = (unsigned)__popcll(wrows), nside = nw + (unsigned)__popcll(erows);
+    // where each row's other cells and its sources start in the two lists: an
+    // inclusive scan of the packed counts (low and high 16 bits) over the rows
+    const unsigned own = (unsigned)__popcll(wl & ~(west | east)) | ((unsigned)__popcll(ws) << 16);
     unsigned incl = own;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -962,15 +977,21 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
         if (lane >= o) incl += t;
     }
     const unsigned all = (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
-    const unsigned n = all & 0xFFFFu, first = incl - own;
-    if (!all && !full) return;  // the workgroup as a whole
+    const unsigned n = nside + (all & 0xFFFFu), first = incl - own;
+    if (!n && !(all >> 16) && !full) return;  // the workgroup as a whole
     if (all >> 16 && threadIdx.x == 0) gbase = atomicAdd(nsrc, all >> 16);
     const unsigned long long below = (1ull << lane) - 1ull;
-    for (int row = w; row < RECON_H; row += NW) {
-        const unsigned long long rl = lane_word(wl, row);
-        const unsigned at = (unsigned)__builtin_amdgcn_readlane((int)first, row) & 0xFFFFu;
+    for (int row = w; row < rows; row += NW) {
+        const unsigned long long rl = lane_word(wl, row), before = (1ull << row) - 1ull;
         const bool on = rl >> lane & 1ull;
-        if (on) list[at + (unsigned)__popcll(rl & below)] = (unsigned short)(row * 64 + lane);
+        unsigned at = (unsigned)__builtin_amdgcn_readlane((int)first, row) & 0xFFFFu;
+        if (west >> lane & 1ull)
+            at = (unsigned)__popcll(wrows & before);
+        else if (east >> lane & 1ull)
+            at = nw + (unsigned)__popcll(erows & before);
+        else
+            at += nside + (unsigned)__popcll(rl & ~(west | east) & below);
+        if (on) list[at] = (unsigned short)(row * 64 + lane);
         if (full && !on && i0 + lane < G.ni && jb + row < G.nj) {
             const size_t c = cix(G, i0 + lane + 1, jb + row + 1);
             O.P.nx[c] = 0.0;
@@ -979,7 +1000,7 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
     }
     __syncthreads();
     if (all >> 16)
-        for (int row = w; row < RECON_H; row += NW) {
+        for (int row = w; row < rows; row += NW) {
             const unsigned long long rs = lane_word(ws, row);
             const unsigned at = (unsigned)__builtin_amdgcn_readlane((int)first, row) >> 16;
             if (rs >> lane & 1ull)
@@ -1721,7 +1742,8 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
     const int ring = 2 * c->ni + 2 * (c->nj - 2);
     const dim3 rblk(256), rgrd((ring + 255) / 256);
     const dim3 pblk(256), pgrd(1024);  // a grid-stride loop over the listed pairs
-    const dim3 rcgrd((c->ni + 63) / 64, (c->nj + RECON_H - 1) / RECON_H);
+    const int rrows = recon_rows((size_t)c->ni * c->nj);
+    const dim3 rcgrd((c->ni + 63) / 64, (c->nj + rrows - 1) / rrows);
     // sweeps: 32x8 tiles (3% faster per transport call than 64x4, 256x1 or
     // 128x2 at 2048^2: the y stencil's rows stay within fewer tiles)
     const dim3 sblk(SWEEP_W, SWEEP_H), sgrd((c->ni + SWEEP_W - 1) / SWEEP_W, (c->nj + SWEEP_H - 1) / SWEEP_H);
@@ -1753,10 +1775,10 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
         constexpr int DIR = decltype(dir)::value;
         const ReconOut O{P, B.fr, B.fl};
         if (scan)
-            hipLaunchKernelGGL((k_recon<DIR, true>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv, full ? 1 : 0,
-                               srcs, nsrc);
+            hipLaunchKernelGGL((k_recon<DIR, true>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv, rrows,
+                               full ? 1 : 0, srcs, nsrc);
         else
-            hipLaunchKernelGGL((k_recon<DIR, false>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv,
+            hipLaunchKernelGGL((k_recon<DIR, false>), rcgrd, dim3(RECON_NT), 0, st, G, v, p, O, bits, dtv, rrows,
                                full ? 1 : 0, srcs, nsrc);
     };
     using std::integral_constant;
