@@ -804,74 +804,101 @@ __device__ __forceinline__ void cell_fluxes(const FluxIn& F, int c, double f, do
     }
 }
 
-// Interface_Reconstruct of cell c: its normal and plane constant where it is an
-// interface cell, then its fluxes.  A three-phase cell whose Ridders search
-// leaves the plane constant unassigned takes the one of the nearest earlier
-// cell in the reference's loop order (i outer, j inner) that assigns it (the
-// reference keeps the previous cell's): the walk back works those cells out
-// again from the same fields, which costs the few lanes that need it a cell's
-// chain more and every other reconstruction nothing.  (As a kernel over a list
-// of such cells it took 3.6 us of each reconstruction at 333 x 171, empty or not.)
+// Interface_Reconstruct of cell c of the lanes with `in`: its normal and plane
+// constant where it is an interface cell, then its fluxes.  A three-phase cell
+// whose Ridders search leaves the plane constant unassigned takes the one of the
+// nearest earlier cell in the reference's loop order (i outer, j inner) that
+// assigns it (the reference keeps the previous cell's).  Those cells are worked
+// out again from the same fields, which costs the wavefronts that hold such a
+// cell another chain or two and every other reconstruction nothing: two steps
+// back each lane on its own, then, as a run of such cells can be as long as a
+// wall, 64 cells at a time for one lane, and for those whose run it is part of.
+// (As a kernel over a list of such cells it took 3.6 us of each reconstruction
+// at 333 x 171, empty or not; with each lane alone, a run of 1024 cells on 256 x
+// 1024 took 3.3 ms of each against 77 us.)
+constexpr int STALE_ALONE = 2;
 template <int DIR>
 __device__ __forceinline__ void recon_cell(const ClsGeo& G, const double* __restrict__ vof,
-                                           const double* __restrict__ phi, const ReconOut& O, double dtv, int c,
-                                           bool full) {
-    int i = c % G.ni + 1, j = c / G.ni + 1;
+                                           const double* __restrict__ phi, const ReconOut& O, double dtv, bool in,
+                                           int c, bool full) {
+    const int lane = __lane_id();
+    const int ci = c % G.ni + 1, cj = c / G.ni + 1;
     double vf = 0.0, vsc = 0.0, hxc = 0.0, hyc = 0.0;
     FluxIn F{};
     double nx = 0.0, ny = 1.0, d = 0.0;
-    bool own = true, itf = false;
-    for (;;) {
-        // everything a two-phase cell may need in one trip to memory
-        const size_t p = cix(G, i, j);
-        int bi, bj;
-        normal_base(G, i, j, bi, bj);
-        const double v = vof[p], vs = G.vofS[p], vsb = G.vofS[cix(G, bi, bj)];
-        const double hx = G.dx[i - 1], hy = G.dy[j - 1];
-        const Stencil S = stencil(G, phi, bi, bj);
-        if (own) {
-            vf = v;
-            vsc = vs;
-            hxc = hx;
-            hyc = hy;
-            if (DIR != FLUX_NONE) {
-                const Line<DIR == FLUX_X> L{G, DIR == FLUX_X ? j : i};
-                const int a = DIR == FLUX_X ? i : j;
-                F = FluxIn{G.nxS[p], G.nyS[p], G.phiS[p], L.vel(a), L.vel(a - 1)};
-            }
-        }
-        const int cl = recon_class(v, vs);
-        bool set = true;
-        if (cl) {
-            double mx, my;
-            if (i == 1 || i == G.ni)
-                final_side(G, vof, phi, i, j, mx, my);
-            else
-                final_inner(G, vof, phi, S, vsb, i, j, mx, my);
-            if (cl == 1)
-                d = plic_distance(v, mx, my, hx, hy);
-            else
-                set = distance_fluid(G.nxS[p], G.nyS[p], G.phiS[p], mx, my, v, hx, hy, d);
+    bool itf = false;
+    int at = (ci - 1) * G.nj + cj - 1;  // the cell to ask next, in the loop's order
+    bool open = in;                     // no plane constant yet
+    for (int round = 0;; ++round) {
+        const unsigned long long left = __ballot(open);
+        if (!left) break;
+        const bool own = round == 0, joint = round > STALE_ALONE;
+        const int top = joint ? __builtin_amdgcn_readlane(at, 63 - __clzll((long long)left)) : 0;
+        const int pos = joint ? top - lane : at;
+        bool set = false;
+        double dp = 0.0;  // before the first cell: the reference's uninitialised local
+        if (joint ? pos >= 0 : open) {
+            const int i = own ? ci : pos / G.nj + 1, j = own ? cj : pos % G.nj + 1;
+            // everything a two-phase cell may need in one trip to memory
+            const size_t p = cix(G, i, j);
+            int bi, bj;
+            normal_base(G, i, j, bi, bj);
+            const double v = vof[p], vs = G.vofS[p], vsb = G.vofS[cix(G, bi, bj)];
+            const double hx = G.dx[i - 1], hy = G.dy[j - 1];
+            const Stencil S = stencil(G, phi, bi, bj);
             if (own) {
-                nx = mx;
-                ny = my;
-                itf = true;
+                vf = v;
+                vsc = vs;
+                hxc = hx;
+                hyc = hy;
+                if (DIR != FLUX_NONE) {
+                    const Line<DIR == FLUX_X> L{G, DIR == FLUX_X ? j : i};
+                    const int a = DIR == FLUX_X ? i : j;
+                    F = FluxIn{G.nxS[p], G.nyS[p], G.phiS[p], L.vel(a), L.vel(a - 1)};
+                }
             }
-        } else {
-            d = default_dis(v, vs, hy);
+            const int cl = recon_class(v, vs);
+            set = true;
+            if (cl) {
+                double mx, my;
+                if (i == 1 || i == G.ni)
+                    final_side(G, vof, phi, i, j, mx, my);
+                else
+                    final_inner(G, vof, phi, S, vsb, i, j, mx, my);
+                if (cl == 1)
+                    dp = plic_distance(v, mx, my, hx, hy);
+                else
+                    set = distance_fluid(G.nxS[p], G.nyS[p], G.phiS[p], mx, my, v, hx, hy, dp);
+                if (own) {
+                    nx = mx;
+                    ny = my;
+                    itf = true;
+                }
+            } else {
+                dp = default_dis(v, vs, hy);
+            }
         }
-        if (set) break;
-        own = false;
-        if (j > 1) {
-            --j;
-        } else if (i > 1) {
-            --i;
-            j = G.nj;
+        if (!joint) {
+            if (open && (set || at == 0)) {
+                d = set ? dp : 0.0;
+                open = false;
+            }
+            --at;
         } else {
-            d = 0.0;  // before the first cell: the reference's uninitialised local
-            break;
+            const unsigned long long hit = __ballot(pos < 0 || set);
+            const int last = hit ? __ffsll((long long)hit) - 1 : 64;  // cells top .. top - last + 1 assign none
+            const double found = __shfl(dp, last & 63, 64);
+            if (open && at <= top && at >= top - last) {
+                if (hit) {
+                    d = found;
+                    open = false;
+                } else {
+                    at = top - 64;
+                }
+            }
         }
     }
+    if (!in) return;
     if (itf || full) {
         O.P.nx[c] = nx;
         O.P.ny[c] = ny;
@@ -1006,10 +1033,11 @@ __global__ void __launch_bounds__(RECON_NT) k_recon(ClsGeo G, const double* __re
             if (rs >> lane & 1ull)
                 srcs[gbase + at + (unsigned)__popcll(rs & below)] = (int)cix(G, i0 + lane + 1, jb + row + 1);
         }
-    for (unsigned t = threadIdx.x; t < n; t += RECON_NT) {
-        const unsigned e = list[t];
+    for (unsigned t0 = w * 64u; t0 < n; t0 += RECON_NT) {
+        const bool in = t0 + lane < n;
+        const unsigned e = in ? list[t0 + lane] : 0u;
         const int c = (int)cix(G, i0 + (int)(e & 63u) + 1, jb + (int)(e >> 6) + 1);
-        recon_cell<DIR>(G, vof, phi, O, dtv, c, full != 0);
+        recon_cell<DIR>(G, vof, phi, O, dtv, in, c, full != 0);
     }
 }
 
