@@ -26,7 +26,8 @@ constexpr int TAIL_MAX = 1024;   // levels with at most this many points run in 
 // threads of the tail, a 2x2 block of its first level each: 256 for up to 256
 // blocks, as on a level of 32 x 32 -- one wavefront per SIMD, so that a
 // thread's couplings, weights and vectors fit its registers in FP64 too -- and
-// 512 for the longer or odd levels, none of which has more blocks
+// 512 for the longer or odd levels, none of which has more blocks; those have
+// half the registers each, and what does not fit stands in LDS (TailArgs)
 constexpr int TAIL_NT = 256, TAIL_NT_MAX = 512;
 constexpr int MAX_TAIL = 10;
 constexpr size_t TAIL_LDS_MAX = 150 * 1024;  // of the tail levels' operators, vectors and weights
@@ -768,8 +769,10 @@ void launch_up5(bool semi, hipStream_t s, Dims F, OpV<T> A, const V* b, const T*
 // A colour pass reads the other colour from one array and writes its own to
 // another, so one barrier ends it.  Sums keep one order of terms and cells,
 // which is the level's and not that of the threads.  At 32 x 32 points, 4 inner
-// iterations, FP64 / FP32: 39 / 39 us; with a thread per cell, every level in
-// LDS and sixteen wavefronts at each barrier, 53 / 56 us.
+// iterations, FP64 / FP32: 42.1 / 39.7 us; with a thread per cell, every level in
+// LDS and sixteen wavefronts at each barrier, 59.9 / 55.4 us.  At 31 x 33, whose
+// 272 blocks take 512 threads: 61.9 / 52.4 us against 78.0 / 71.5 (82.4 / 59.9 with
+// all weights in registers, of which the compiler spilled 210 / 8).
 enum { TA_D = 0, TA_E, TA_N, TA_NE, TA_NW, TA_X, TA_B, TA_R, TA_COUNT };
 
 template <typename T>
@@ -795,7 +798,17 @@ struct TailArgs {
     int ld0, x0, x1;  // level 0's arrays XA, XB: element (i, j) at (j + 1) * ld0 + i + 1
     int ld1, y0, y1;  // level 1's arrays YA, YB, likewise
     int lin;          // three level 0 vectors in linear order (inner iterations)
+    int n1;           // points of level 1, the threads with a block
+    // TAIL_NT_MAX threads: weights in LDS, nine planes each, of the restriction to
+    // level 2 and (tail_staged) of the restriction from a block and the
+    // prolongation to it
+    int w2, rw1, pw1;
 };
+
+// whether TAIL_NT_MAX threads keep the weights between the first two levels in LDS:
+// at most 114 KB with them on any level that fits the budget, 88 KB in FP32 without
+template <typename T>
+constexpr bool tail_staged = sizeof(T) == 8;
 
 // offset of cell (i,j) in the LDS arrays of a level >= 2 (compact layout)
 __device__ inline int toff(const Dims& D, int i, int j) { return (j + 2) * D.ld + i; }
@@ -1166,9 +1179,10 @@ __device__ __forceinline__ void tail_level2(T* lds, const TailArgs<T>& a, const 
 // One V-cycle over the tail levels: b -> x on the thread's block.  lower: how
 // the levels 2.. run (TAIL_LOWER_*).
 enum { TAIL_LOWER_ALL = 0, TAIL_LOWER_WAVE, TAIL_LOWER_OWN };
-template <typename T>
+template <int NT, typename T>
 __device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const TailOwn<T>& O, const double* inv,
                                             int lower, const T (&b)[4], T (&x)[4]) {
+    constexpr bool MANY = NT > TAIL_NT, STAGED = MANY && tail_staged<T>;
     const int tid = threadIdx.x;
     T* XA = lds + a.x0;
     T* XB = lds + a.x1;
@@ -1177,7 +1191,7 @@ __device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const 
     const int ld = a.ld0, ld1 = a.ld1;
     T* xa = XA + O.p;
     T* xb = XB + O.p;
-    if (a.n == 1) {
+    if (!MANY && a.n == 1) {
         // the first tail level is the coarsest
         const Dims& D = a.L[0].d;
         if (O.own) {
@@ -1232,12 +1246,15 @@ __device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const 
     T* ya = YA + O.p1;
     T* yb = YB + O.p1;
     if (O.own) {
-        b1 = O.rw[0] * r[0];
-        b1 += O.rw[1] * r[1] + O.rw[2] * xb[-1];
-        b1 += O.rw[3] * r[2] + O.rw[4] * xb[-ld];
-        b1 += O.rw[5] * r[3] + O.rw[6] * xb[ld - 1] + O.rw[7] * xb[1 - ld] + O.rw[8] * xb[-ld - 1];
+        T w[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = STAGED ? lds[a.rw1 + k * a.n1 + tid] : O.rw[k];
+        b1 = w[0] * r[0];
+        b1 += w[1] * r[1] + w[2] * xb[-1];
+        b1 += w[3] * r[2] + w[4] * xb[-ld];
+        b1 += w[5] * r[3] + w[6] * xb[ld - 1] + w[7] * xb[1 - ld] + w[8] * xb[-ld - 1];
     }
-    if (a.n == 2) {
+    if (!MANY && a.n == 2) {
         const Dims& D = a.L[1].d;
         if (O.own) ya[0] = b1;
         __syncthreads();
@@ -1261,10 +1278,14 @@ __device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const 
         T b2 = T(0);
         if (O.c2 >= 0) {
             const T* f = YB + O.f2;
-            b2 = O.rw2[0] * f[0];
-            b2 += O.rw2[1] * f[1] + O.rw2[2] * f[-1];
-            b2 += O.rw2[3] * f[ld1] + O.rw2[4] * f[-ld1];
-            b2 += O.rw2[5] * f[ld1 + 1] + O.rw2[6] * f[ld1 - 1] + O.rw2[7] * f[1 - ld1] + O.rw2[8] * f[-ld1 - 1];
+            const int n2 = L2.d.ni * L2.d.nj;
+            T w[9];
+#pragma unroll
+            for (int k = 0; k < 9; ++k) w[k] = MANY ? lds[a.w2 + k * n2 + tid] : O.rw2[k];
+            b2 = w[0] * f[0];
+            b2 += w[1] * f[1] + w[2] * f[-1];
+            b2 += w[3] * f[ld1] + w[4] * f[-ld1];
+            b2 += w[5] * f[ld1 + 1] + w[6] * f[ld1 - 1] + w[7] * f[1 - ld1] + w[8] * f[-ld1 - 1];
             if (lower != TAIL_LOWER_OWN) tarr(lds, L2, TA_B)[O.c2] = b2;
         }
         if (lower == TAIL_LOWER_OWN) {
@@ -1313,10 +1334,13 @@ __device__ __forceinline__ void tail_vcycle(T* lds, const TailArgs<T>& a, const 
     // level 0 up: correction, black, red
     if (O.own) {
         const T e00 = yb[0], e10 = yb[1], e01 = yb[ld1], e11 = yb[ld1 + 1];
-        x[0] = corrected(x[0], O.pw[0] * e00);
-        x[1] = corrected(x[1], O.pw[1] * e00 + O.pw[2] * e10);
-        x[2] = corrected(x[2], O.pw[3] * e00 + O.pw[4] * e01);
-        x[3] = corrected(x[3], O.pw[5] * e00 + O.pw[6] * e10 + O.pw[7] * e01 + O.pw[8] * e11);
+        T w[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = STAGED ? lds[a.pw1 + k * a.n1 + tid] : O.pw[k];
+        x[0] = corrected(x[0], w[0] * e00);
+        x[1] = corrected(x[1], w[1] * e00 + w[2] * e10);
+        x[2] = corrected(x[2], w[3] * e00 + w[4] * e01);
+        x[3] = corrected(x[3], w[5] * e00 + w[6] * e10 + w[7] * e01 + w[8] * e11);
         xa[0] = x[0];
         xa[1] = x[1];
         xa[ld] = x[2];
@@ -1357,6 +1381,9 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
     __shared__ double part_b[TAIL_GROUPS][2];
     __shared__ double part_a[TAIL_GROUPS][2];
     T* lds = reinterpret_cast<T*>(smem_raw);
+    // more than 256 blocks are as many points on level 1 and more than 64 on
+    // level 2: there is a level 2, and the whole workgroup runs it
+    constexpr bool MANY = NT > TAIL_NT, STAGED = MANY && tail_staged<T>;
     const int tid = threadIdx.x;
     const int live = a.on ? *a.on : 1;
     // everything the passes read from memory, asked for before the flag is looked at
@@ -1377,7 +1404,7 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
             O.r[k] = tail_row(L0, i, j);
             if (i < D0.ni && j < D0.nj) b[k] = L0.b[D0.off(i, j)];
         }
-        if (a.n > 1) {
+        if (!STAGED && a.n > 1) {
             const Dims& D1 = a.L[1].d;
             restrict_weights(D1, L0.P, I, J, O.rw);
 #pragma unroll
@@ -1404,10 +1431,10 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
     if (a.n > 2) {
         const Dims& D2 = a.L[2].d;
         const int n2 = D2.ni * D2.nj;
-        if (n2 <= 64) lower = a.n == 4 ? TAIL_LOWER_OWN : TAIL_LOWER_WAVE;
+        if (!MANY && n2 <= 64) lower = a.n == 4 ? TAIL_LOWER_OWN : TAIL_LOWER_WAVE;
         const int I2 = tid % D2.ni, J2 = tid / D2.ni;
         if (J2 < D2.nj) {
-            restrict_weights(D2, a.L[1].P, I2, J2, O.rw2);
+            if (!MANY) restrict_weights(D2, a.L[1].P, I2, J2, O.rw2);
             O.c2 = toff(a.L[2].cd, I2, J2);
             O.f2 = (2 * J2 + 1) * a.ld1 + 2 * I2 + 1;
             O.red2 = ((I2 + J2) & 1) == 0;
@@ -1422,6 +1449,23 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
         for (int k = tid; k < nc * nc; k += NT) inv[k] = a.inv[k];
     }
     __syncthreads();
+    if (STAGED && O.own) {
+        const Dims& D1 = a.L[1].d;
+        T w[9];
+        restrict_weights(D1, L0.P, I, J, w);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            lds[a.rw1 + k * a.n1 + tid] = w[k];
+            lds[a.pw1 + k * a.n1 + tid] = L0.P.w[k][D1.off(I, J)];
+        }
+    }
+    if (MANY && O.c2 >= 0) {
+        const Dims& D2 = a.L[2].d;
+        T w[9];
+        restrict_weights(D2, a.L[1].P, tid % D2.ni, tid / D2.ni, w);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) lds[a.w2 + k * D2.ni * D2.nj + tid] = w[k];
+    }
     // operators and weights of the levels 2..
     for (int l = 2; l < a.n; ++l) {
         const TailLevel<T>& L = a.L[l];
@@ -1450,7 +1494,7 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
     __syncthreads();
     T x[4] = {T(0), T(0), T(0), T(0)};
     if (a.krylov <= 0) {
-        tail_vcycle(lds, a, O, inv, lower, b, x);
+        tail_vcycle<NT>(lds, a, O, inv, lower, b, x);
     } else {
         // b holds the inner residual; the level's vectors z, q, p and b go to
         // LDS in linear order for the dots
@@ -1474,7 +1518,7 @@ __global__ void __launch_bounds__(NT) k_tail(TailArgs<T> a, int lds_elems) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) z[k] = T(0);
             store(bl, b);
-            tail_vcycle(lds, a, O, inv, lower, b, z);
+            tail_vcycle<NT>(lds, a, O, inv, lower, b, z);
             store(zl, z);
             __syncthreads();
             double v[2];
@@ -1610,6 +1654,11 @@ int tail_layout(Ctx* c, int lt, const int* on, TailArgs<T>& ta, size_t& lds) {
     ta.y0 = take(ta.ld1 * (cj + 2));
     ta.y1 = take(ta.ld1 * (cj + 2));
     ta.lin = take(ta.krylov > 0 ? 3 * TAIL_MAX : 0);
+    ta.n1 = ci * cj;
+    const bool many = ta.n1 > TAIL_NT;
+    ta.w2 = take(many ? 9 * c->lev[lt + 2].d.ni * c->lev[lt + 2].d.nj : 0);
+    ta.rw1 = take(many && tail_staged<T> ? 9 * ta.n1 : 0);
+    ta.pw1 = take(many && tail_staged<T> ? 9 * ta.n1 : 0);
     size_t all = ta.krylov > 0 ? compact(d0).alloc_elems() : 0;
     for (int k = 0; k < ta.n; ++k) {
         const Level& L = c->lev[lt + k];
@@ -1676,16 +1725,11 @@ int vcycle(Ctx* c, const V* r, V* z, const V* q, Slots S, int* dots_done, const 
     size_t tail_lds = 0;
     int rc = tail_layout<T>(c, lt, on, ta, tail_lds);
     if (rc) return rc;
-    {
-        const Dims& d = c->lev[lt].d;
-        const int blocks = ((d.ni + 1) / 2) * ((d.nj + 1) / 2);
-        if (blocks <= TAIL_NT)
-            hipLaunchKernelGGL((k_tail<T, TAIL_NT>), dim3(1), dim3(TAIL_NT), tail_lds * sizeof(T), s, ta,
-                               (int)tail_lds);
-        else
-            hipLaunchKernelGGL((k_tail<T, TAIL_NT_MAX>), dim3(1), dim3(TAIL_NT_MAX), tail_lds * sizeof(T), s, ta,
-                               (int)tail_lds);
-    }
+    if (ta.n1 <= TAIL_NT)
+        hipLaunchKernelGGL((k_tail<T, TAIL_NT>), dim3(1), dim3(TAIL_NT), tail_lds * sizeof(T), s, ta, (int)tail_lds);
+    else
+        hipLaunchKernelGGL((k_tail<T, TAIL_NT_MAX>), dim3(1), dim3(TAIL_NT_MAX), tail_lds * sizeof(T), s, ta,
+                           (int)tail_lds);
     // up: level l reads x_l from the down pass and e_{l+1}; writes its own
     // correction into r_l (its solution for the level above)
     for (int l = lt - 1; l >= 0; --l) {

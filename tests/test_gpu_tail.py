@@ -74,6 +74,17 @@ def test_tail_of_any_shape(oracle_lib, ni, nj, solid, precision):
     assert its[4] <= its[0] + 1
 
 
+@pytest.mark.parametrize("ni,nj,solid,precision", [
+    (58, 70, True, 0), (58, 70, False, 1),    # 29 x 35: 270 blocks, of which the last hang over both edges
+    (18, 216, True, 0), (18, 216, False, 1),  # 9 x 108: the largest LDS of FP64, third level of 81 points
+    (2, 1400, False, 1),                      # 1 x 700: 350 blocks, third level of 175 points (FP32 only)
+])
+def test_tail_of_more_than_256_blocks(oracle_lib, ni, nj, solid, precision):
+    """The levels that take 512 threads, whose weights to level 2, and in FP64
+    between the first two levels, stand in LDS."""
+    test_tail_of_any_shape(oracle_lib, ni, nj, solid, precision)
+
+
 @pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
 @pytest.mark.parametrize("ni,nj", [(64, 64), (60, 34), (128, 96), (37, 75)])
 def test_all_neumann(ni, nj, precision):
