@@ -484,18 +484,17 @@ __global__ void __launch_bounds__(256) k_poolT_add_mask(T4 dd, T4 skip, T4 act, 
 }
 
 // loss = sum mask*(y-t)^2 / n ; gout channel 0 = 2 mask (y-t) / n.  A workgroup
-// takes LOSS_PX pixels: bound by the adds to the one sum, one a workgroup (256
-// pixels each: 57.6 us at 16 x 256 x 256 pixels; 2048: 22.7).
-constexpr int LOSS_PX = 2048;
+// takes `per` times 256 pixels: a large batch is bound by the adds to the one sum,
+// one a workgroup (16 x 256 x 256 pixels, 256 each: 57.6 us; 2048: 21.9), a small
+// one by the chain of a thread's pixels (16 x 128, 256 each: 3.5 us; 2048: 8.6).
 __global__ void __launch_bounds__(256) k_loss(const float* __restrict__ y, const float* __restrict__ t,
-                                              const float* __restrict__ m, T4 g, int nb, float inv_n,
+                                              const float* __restrict__ m, T4 g, int nb, float inv_n, int per,
                                               float* __restrict__ loss) {
     __shared__ float red[4];
     const long n = (long)nb * g.H * g.W;
     float l = 0.f;
-#pragma unroll
-    for (int k = 0; k < LOSS_PX / 256; ++k) {
-        const long e = (long)blockIdx.x * LOSS_PX + k * 256 + threadIdx.x;
+    for (int k = 0; k < per; ++k) {
+        const long e = ((long)blockIdx.x * per + k) * 256 + threadIdx.x;
         if (e >= n) break;
         const int x = (int)(e % g.W);
         const long r = e / g.W;
@@ -803,8 +802,10 @@ int backward(Net* n, const bf16* Xp, const float* t, const float* mask, int nb) 
     hipLaunchKernelGGL(k_fill, dim3(blocks((long)n->nw)), dim3(256), 0, s, n->g, n->nw, 0.f);
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(256), 0, s, n->loss, (size_t)1, 0.f);
     const long npx = (long)nb * n->H * n->W;
-    hipLaunchKernelGGL(k_loss, dim3((unsigned)((npx + LOSS_PX - 1) / LOSS_PX)), dim3(256), 0, s, (const float*)n->y, t, mask, n->gout, nb,
-                       1.f / (float)npx, n->loss);
+    // a workgroup a CU before any takes more than its first 256 pixels
+    const int per = (int)std::clamp(npx / (256 * 256), 1l, 8l);
+    hipLaunchKernelGGL(k_loss, dim3((unsigned)((npx + 256 * per - 1) / (256 * per))), dim3(256), 0, s,
+                       (const float*)n->y, t, mask, n->gout, nb, 1.f / (float)npx, per, n->loss);
     auto upT = [&](T4 d, T4 act, T4 P) {
         hipLaunchKernelGGL(k_upT_mask, dim3(blocks((long)nb * P.H * P.W * (P.C / 8))), dim3(256), 0, s, d, act, P,
                            nb);
