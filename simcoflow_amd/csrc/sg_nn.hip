@@ -275,33 +275,39 @@ __device__ __forceinline__ bf16x8 transpose8(const bf16x8& v) {
 // transposes for 9 * MBW MFMAs, the next row's loads in flight meanwhile, and
 // no barrier until the strip ends.  Waves of a workgroup with the same channels
 // add up in LDS before their atomics.  Measured at 16 x 256 x 256 pixels, 16 x
-// 16 channels: 29 us for 67 MB, 2.3 TB/s; one tap a workgroup, with 32-pixel
+// 16 channels: 28 us for 67 MB, 2.4 TB/s; one tap a workgroup, with 32-pixel
 // tiles transposed through LDS by 2-byte writes and two barriers a tile, took
 // 254 us.
+//
+// TR: the tap rows a wave takes, all 3, or 1 (blockIdx.y) on levels too small to
+// fill the chip: a third of the chain of transposes and sums, for three times the
+// loads and waves.  16 x 16 channels at 16 x 128 pixels: 3.6 us, 5.9 with all
+// three tap rows, 10.1 with those and strips no shorter than 8 rows.
 template <int CIN, int COUT>
 struct DwSplit {
     static constexpr int MBW = COUT >= 32 ? 2 : 1;
     static constexpr int NBK = (CIN + 15) / 16;
     static constexpr int PAIRS = COUT / 16 / MBW * NBK;  // (output, input) channel groups
 };
-template <int CIN, int COUT>
+template <int CIN, int COUT, int TR>
 __global__ void __launch_bounds__(256) k_dw(T4 X, T4 P, float* __restrict__ dW, int nb, int rows) {
     using S = DwSplit<CIN, COUT>;
     constexpr int MBW = S::MBW, KP = kpad(CIN), PAIRS = S::PAIRS;
     constexpr int PB = PAIRS < 4 ? PAIRS : 4;  // channel groups in a workgroup
     constexpr int SHARE = 4 / PB;              // waves of a workgroup with the same one
-    constexpr int NACC = 9 * MBW * 4;
+    constexpr int TAPS = 3 * TR, NACC = TAPS * MBW * 4;
     static_assert(PAIRS < 4 ? 4 % PAIRS == 0 : PAIRS % 4 == 0, "waves must divide among the channel groups");
-    __shared__ float sum[SHARE > 1 ? PB * NACC * 64 : 1];
+    __shared__ float part[SHARE > 1 ? 4 * NACC * 64 : 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, r16 = lane & 15, q4 = lane >> 4;
     const long wid = (long)blockIdx.x * 4 + wv;
     const int pair = (int)(wid % PAIRS);
     const long strip = wid / PAIRS;
     const int c0 = pair % S::NBK * 16, co0 = pair / S::NBK * (16 * MBW);
     const int chunks = (P.W + 31) / 32, segs = (P.H + rows - 1) / rows;
-    floatx4 acc[9][MBW];
+    const int dy0 = TR == 1 ? (int)blockIdx.y : 0;
+    floatx4 acc[TAPS][MBW];
 #pragma unroll
-    for (int k = 0; k < 9; ++k)
+    for (int k = 0; k < TAPS; ++k)
 #pragma unroll
         for (int m = 0; m < MBW; ++m) acc[k][m] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (strip < (long)nb * segs * chunks) {
@@ -313,83 +319,100 @@ __global__ void __launch_bounds__(256) k_dw(T4 X, T4 P, float* __restrict__ dW, 
         // pixels past the row's end and channels past the last one read as zero
         const bool okp = x < P.W, okx = okp && c0 + half < CIN;
         const bf16* pp = P.p + t4off(P, b, y0 + 1, okp ? x + 1 : 0) + co0 + half;
-        const bf16* px = X.p + t4off(X, b, y0, okx ? x : 0) + c0 + (okx ? half : 0);
+        const bf16* px = X.p + t4off(X, b, y0 + dy0, okx ? x : 0) + c0 + (okx ? half : 0);
         const long ps = (long)(P.W + 2) * COUT, xs = (long)(X.W + 2) * CIN;
         const bf16x8 zero = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
         bf16x8 rx[3], rp[MBW], xr[3][3];
-        auto load_x = [&](int row) {
+        auto load_x = [&](int row, bf16x8 (&to)[3]) {
 #pragma unroll
-            for (int d = 0; d < 3; ++d) rx[d] = okx ? *(const bf16x8*)(px + row * xs + d * CIN) : zero;
+            for (int d = 0; d < 3; ++d) to[d] = okx ? *(const bf16x8*)(px + row * xs + d * CIN) : zero;
         };
         auto load_p = [&](int row) {
 #pragma unroll
             for (int m = 0; m < MBW; ++m) rp[m] = okp ? *(const bf16x8*)(pp + row * ps + 16 * m) : zero;
         };
-        auto turn_x = [&](bf16x8 (&to)[3]) {
+        auto turn_x = [&](const bf16x8 (&from)[3], bf16x8 (&to)[3]) {
 #pragma unroll
-            for (int d = 0; d < 3; ++d) to[d] = transpose8(rx[d]);
+            for (int d = 0; d < 3; ++d) to[d] = transpose8(from[d]);
         };
-        load_x(0);
-        turn_x(xr[0]);
-        load_x(1);
-        turn_x(xr[1]);
-        load_x(2);
-        load_p(0);
         const int n = y1 - y0;
-        // row r of the strip: X rows r, r + 1, r + 2 sit in xr[i], xr[i + 1], xr[i + 2] (mod 3)
-        auto row = [&](int r, bf16x8 (&xa)[3], bf16x8 (&xb)[3], bf16x8 (&xc)[3]) {
-            if (r >= n) return;
-            turn_x(xc);
-            bf16x8 pa[MBW];
+        auto turn_p = [&](bf16x8 (&to)[MBW]) {
 #pragma unroll
-            for (int m = 0; m < MBW; ++m) pa[m] = transpose8(rp[m]);
-            if (r + 1 < n) {
-                load_x(r + 3);
-                load_p(r + 1);
-            }
-#pragma unroll
-            for (int m = 0; m < MBW; ++m)
-#pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    acc[d][m] = mfma(pa[m], xa[d], acc[d][m]);
-                    acc[3 + d][m] = mfma(pa[m], xb[d], acc[3 + d][m]);
-                    acc[6 + d][m] = mfma(pa[m], xc[d], acc[6 + d][m]);
-                }
+            for (int m = 0; m < MBW; ++m) to[m] = transpose8(rp[m]);
         };
-        for (int r = 0; r < n; r += 3) {
-            row(r, xr[0], xr[1], xr[2]);
-            row(r + 1, xr[1], xr[2], xr[0]);
-            row(r + 2, xr[2], xr[0], xr[1]);
+        if constexpr (TR == 3) {
+            load_x(0, xr[0]);
+            load_x(1, xr[1]);
+            load_x(2, rx);
+            load_p(0);
+            turn_x(xr[0], xr[0]);
+            turn_x(xr[1], xr[1]);
+            // row r of the strip: X rows r, r + 1, r + 2 sit in xr[i], xr[i + 1], xr[i + 2] (mod 3)
+            auto row = [&](int r, bf16x8 (&xa)[3], bf16x8 (&xb)[3], bf16x8 (&xc)[3]) {
+                if (r >= n) return;
+                turn_x(rx, xc);
+                bf16x8 pa[MBW];
+                turn_p(pa);
+                if (r + 1 < n) {
+                    load_x(r + 3, rx);
+                    load_p(r + 1);
+                }
+#pragma unroll
+                for (int m = 0; m < MBW; ++m)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) {
+                        acc[d][m] = mfma(pa[m], xa[d], acc[d][m]);
+                        acc[3 + d][m] = mfma(pa[m], xb[d], acc[3 + d][m]);
+                        acc[6 + d][m] = mfma(pa[m], xc[d], acc[6 + d][m]);
+                    }
+            };
+            for (int r = 0; r < n; r += 3) {
+                row(r, xr[0], xr[1], xr[2]);
+                row(r + 1, xr[1], xr[2], xr[0]);
+                row(r + 2, xr[2], xr[0], xr[1]);
+            }
+        } else {
+            load_x(0, rx);
+            load_p(0);
+            for (int r = 0; r < n; ++r) {
+                bf16x8 pa[MBW];
+                turn_x(rx, xr[0]);
+                turn_p(pa);
+                if (r + 1 < n) {
+                    load_x(r + 1, rx);
+                    load_p(r + 1);
+                }
+#pragma unroll
+                for (int m = 0; m < MBW; ++m)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) acc[d][m] = mfma(pa[m], xr[0][d], acc[d][m]);
+            }
         }
     }
     auto put = [&](int k, int m, int r, int ln, int pr, float v) {
         const int ci = pr % S::NBK * 16 + (ln & 15);
         const int co = pr / S::NBK * (16 * MBW) + m * 16 + 4 * (ln >> 4) + r;
-        if (ci < CIN) atomicAdd(dW + (size_t)co * KP + k * CIN + ci, v);
+        if (ci < CIN) atomicAdd(dW + (size_t)co * KP + (3 * dy0 + k) * CIN + ci, v);
     };
     if constexpr (SHARE > 1) {
-        float* mine = sum + (size_t)(wv % PB) * NACC * 64 + lane;
-        for (int w = 0; w < SHARE; ++w) {
-            if (wv / PB == w) {
+        float* mine = part + wv * NACC * 64 + lane;
 #pragma unroll
-                for (int k = 0; k < 9; ++k)
+        for (int k = 0; k < TAPS; ++k)
 #pragma unroll
-                    for (int m = 0; m < MBW; ++m)
+            for (int m = 0; m < MBW; ++m)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            float* s = mine + ((k * MBW + m) * 4 + r) * 64;
-                            *s = w ? *s + acc[k][m][r] : acc[k][m][r];
-                        }
-            }
-            __syncthreads();
-        }
+                for (int r = 0; r < 4; ++r) mine[((k * MBW + m) * 4 + r) * 64] = acc[k][m][r];
+        __syncthreads();
         for (int e = tid; e < PB * NACC * 64; e += 256) {
             const int ln = e & 63, q = e >> 6, i = q % NACC;
-            put(i / (4 * MBW), i / 4 % MBW, i % 4, ln, q / NACC, sum[e]);
+            float v = part[e];
+#pragma unroll
+            for (int w = 1; w < SHARE; ++w) v += part[w * PB * NACC * 64 + e];
+            put(i / (4 * MBW), i / 4 % MBW, i % 4, ln, q / NACC, v);
         }
     } else {
 #pragma unroll
-        for (int k = 0; k < 9; ++k)
+        for (int k = 0; k < TAPS; ++k)
 #pragma unroll
             for (int m = 0; m < MBW; ++m)
 #pragma unroll
@@ -610,17 +633,37 @@ int conv(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb, int ep
     return SG_OK;
 }
 
-constexpr long DW_WAVES = 2048;
+// Strips of as many rows as leave DW_WAVES waves, two a SIMD, where the level is
+// large enough; below, strips down to one row high as long as there are no more
+// than DW_ROW of them, from which on a strip's two rows of X beyond its own and its
+// atomics cost more than its shorter chain gains: the least of a sweep of 64 to
+// 320.  From DW_SPLIT strips of one row on, a wave takes all three tap rows.
+// A gradient, us, split below 512 / 1024 / 2048 / 4096 / 8192 / 16384 such strips (and
+// with the kernel of one tap a workgroup):
+//   16 x 128                 412: 410 / 412 / 412 / 412 / 412 (420)
+//   128 x 128                465: 462 / 462 / 460 / 462 / 463 (540)
+//   200 x 256                555: 537 / 528 / 525 / 525 / 525 (720)
+//   6 x 64 x 256             660: 652 / 637 / 621 / 626 / 623 (993)
+//   8 x 128 x 256            853: 853 / 840 / 841 / 868 / 884 (1500)
+//   16 x 256 x 256           1627: 1626 / 1626 / 1628 / 1643 / 1764 (3630)
+constexpr long DW_WAVES = 2048, DW_ROW = 160, DW_SPLIT = 4096;
+
+template <int CIN, int COUT, int TR>
+void dw_launch(Net* n, int l, T4 X, T4 P, int nb, int rows, long lines) {
+    const long waves = lines * ((P.H + rows - 1) / rows);
+    hipLaunchKernelGGL((k_dw<CIN, COUT, TR>), dim3((unsigned)((waves + 3) / 4), 3 / TR), dim3(256), 0, n->stream, X, P,
+                       n->g + n->woff[l], nb, rows);
+}
 
 template <int CIN, int COUT>
 int dw(Net* n, int l, T4 X, T4 P, int nb) {
-    // rows per strip: two waves per SIMD where the level is large enough, no
-    // shorter than 8 rows (a strip reads two rows of X beyond its own)
-    const long pairs = DwSplit<CIN, COUT>::PAIRS, chunks = (P.W + 31) / 32;
-    const int rows = (int)std::max(8l, nb * P.H * chunks * pairs / DW_WAVES);
-    const long waves = nb * ((P.H + rows - 1) / rows) * chunks * pairs;
-    hipLaunchKernelGGL((k_dw<CIN, COUT>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, n->stream, X, P,
-                       n->g + n->woff[l], nb, rows);
+    const long lines = nb * (long)((P.W + 31) / 32) * DwSplit<CIN, COUT>::PAIRS;
+    const long one = lines * P.H;  // strips one row high
+    const int rows = (int)std::max(std::clamp(one / DW_ROW, 1l, 8l), one / DW_WAVES);
+    if (one < DW_SPLIT)
+        dw_launch<CIN, COUT, 1>(n, l, X, P, nb, rows, lines);
+    else
+        dw_launch<CIN, COUT, 3>(n, l, X, P, nb, rows, lines);
     SG_HIP(hipGetLastError());
     return SG_OK;
 }

@@ -67,3 +67,22 @@ def test_weight_gradient_of_long_strips():
     # the output gradient is rounded to BF16 after the division by the number
     # of points, a power of two here, so the halves round alike
     assert _rel(whole.astype(np.float64), mean) <= 6e-5
+
+
+@pytest.mark.parametrize("H,W,copies", [(8, 128, 128), (16, 128, 64), (64, 128, 16), (24, 384, 16), (72, 256, 8)])
+def test_weight_gradient_of_an_image_and_of_its_copies(H, W, copies):
+    """An image alone has so few strips that a wave takes one row of taps, in strips
+    of one row and a few; a batch of its copies has 4096 of a row or more on the
+    finest level, whose waves take all nine taps, and longer ones below.  The loss is
+    a mean, so the gradients are equal: the copies' number is a power of two, so the
+    output gradient rounds alike, and both take the same convolutions.  What is left
+    is the order of FP32 sums of at most 1.5e5 terms: 4e2 * 6e-8 = 2.4e-5 (the loss,
+    added up by workgroups of other sizes, likewise)."""
+    from simcoflow_amd.learned import init_weights
+    print(f"[nn] weight gradient H={H} W={W}, {copies} copies", flush=True)
+    w = init_weights(4)
+    x, t, m = _batch(H, W, 1, 5)
+    one, loss = _gradient(H, W, 1, w, x, t, m)
+    many, loss_many = _gradient(H, W, copies, w, *(np.repeat(a, copies, axis=0) for a in (x, t, m)))
+    assert _rel(many.astype(np.float64), one.astype(np.float64)) <= 2.4e-5
+    assert abs(float(loss_many) - float(loss)) <= 2.4e-5 * float(loss)
