@@ -130,11 +130,12 @@ __global__ void __launch_bounds__(256) k_conv(T4 in, const bf16* __restrict__ wt
 // Chunks of the reduction do not run over the end of a tap row: 3 x 8 channels
 // fill 24 of 32, 3 x 16 take two chunks.
 //
-// At 16 images, us a layer against k_conv: 16 x 16 at 256^2 24.4 / 26.4, 32 x 16
-// 30.6 / 41.2, 32 x 32 at 128^2 18.3 / 21.5, 64 x 32 40.9 / 37.2 forward with the
-// skip, 64 x 64 at 64^2 22.8 / 28.5, 128 x 64 40.0 / 51.9, 128 x 128 at 32^2 30.3 /
-// 43.0.  The narrow layers are bound by their activations' bytes (2.7 TB/s at 24.4
-// us), the wide ones by the loads' latency at two waves a SIMD.
+// At 16 images, us a layer against k_conv: 16 x 16 at 256^2 24.1 / 26.6, 32 x 16
+// 30.3 / 40.4, 32 x 32 at 128^2 18.1 / 20.9, 32 x 64 25.3 / 42.0, 64 x 32 (with the
+// skip) 40.5 / 57, 64 x 64 at 64^2 22.5 / 28.5, 128 x 64 39.9 / 52.2, 64 x 128 34.6 /
+// 41.4, 128 x 128 at 32^2 30.1 / 42.7.  The narrow layers are bound by their
+// activations' bytes (2.7 TB/s at 24.1 us), the wide ones by the loads' latency at two
+// waves a SIMD.
 template <int CIN>
 struct StripK {
     static constexpr int FR = CIN == 8 ? 1 : CIN == 16 ? 2 : 3 * CIN / 32;  // chunks of a tap row
@@ -599,9 +600,12 @@ void conv_split(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb,
 // 8192 a 16 x 16 layer of 16 x 256 x 256 pixels takes 26.5 and 28.1 us against
 // 24.4, a 32 x 32 one of 16 x 128 x 128 22.7 and 22.7 against 18.3.  64-pixel
 // strips where those can be two rows high; else, for the layers whose work per
-// pixel is large, 32-pixel ones (64 x 64 at 16 x 64 x 64: 22.8 against 27.6 us),
-// one row high if need be (128 x 128 at 16 x 32 x 32: 30.3 against k_conv's 43.0).
-// With fewer tiles k_conv, which splits the channels further, keeps the chip fuller.
+// pixel is large, 32-pixel ones (64 x 64 at 16 x 64 x 64: 22.5 against 28.5 us),
+// one row high if need be (128 x 128 at 16 x 32 x 32: 30.1 against k_conv's 42.7)
+// where the channels come to 64 or more (64 x 32 at 16 x 64 x 64: 17.3 against
+// 16.5).  With fewer tiles k_conv, which splits the channels further, keeps the chip
+// fuller.  Layers of fewer channels are on the two finest levels only, whose widths
+// are multiples of 64.
 constexpr long STRIP_WAVES = 2048;
 
 template <int CIN, int COUT, int MB, int NPB>
@@ -619,8 +623,12 @@ bool conv_strip(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb,
 template <int CIN, int COUT>
 int conv(Net* n, T4 in, const bf16* w, T4 out, T4 aux, float* yo, int nb, int epi) {
     constexpr int MB = COUT == 16 ? 1 : 2;
-    if ((CIN < 128 && conv_strip<CIN, COUT, MB, (CIN < 128 ? 4 : 2)>(n, in, w, out, aux, yo, nb, epi, 2 * STRIP_WAVES)) ||
-        ((CIN >= 64 || in.W % 64) && conv_strip<CIN, COUT, MB, 2>(n, in, w, out, aux, yo, nb, epi, STRIP_WAVES))) {
+    bool strip = false;
+    if constexpr (CIN < 128) strip = conv_strip<CIN, COUT, MB, 4>(n, in, w, out, aux, yo, nb, epi, 2 * STRIP_WAVES);
+    if constexpr (CIN >= 64 || COUT >= 64)
+        if (!strip && (CIN >= 64 || in.W % 64))
+            strip = conv_strip<CIN, COUT, MB, 2>(n, in, w, out, aux, yo, nb, epi, (COUT >= 64 ? 1 : 2) * STRIP_WAVES);
+    if (strip) {
         SG_HIP(hipGetLastError());
         return SG_OK;
     }
