@@ -1814,17 +1814,19 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
     const integral_constant<int, FLUX_X> flux_x{};
     const integral_constant<int, FLUX_Y> flux_y{};
     // sg_sweep_timing: an event before (end = 0) and after (end = 1) each sweep
+    // (waiting for those before it when the pool is used up, wherever that is in a call)
     auto& TM = c->sweep_timing;
-    if (TM.on && TM.used + 2 * nsub > Ctx::SweepTiming::POOL) {
-        const int rc = sweep_timing_drain(c);
-        if (rc) return rc;
-    }
-    auto sweep_mark = [&](int end) -> hipError_t {
-        if (!TM.on) return hipSuccess;
-        const hipError_t e = hipEventRecord(TM.ev[2 * TM.used + end], st);
+    auto sweep_mark = [&](int end) -> int {
+        if (!TM.on) return SG_OK;
+        if (!end && TM.used == Ctx::SweepTiming::POOL) {
+            const int rc = sweep_timing_drain(c);
+            if (rc) return rc;
+        }
+        SG_HIP(hipEventRecord(TM.ev[2 * TM.used + end], st));
         if (end) ++TM.used;
-        return e;
+        return SG_OK;
     };
+    int rc = SG_OK;
     for (int k = 1; k <= nsub; ++k) {
         // first sweep: (vof, phi) -> (vt, pt), implicit divergence; after the
         // first sub-step the bits are those of the last reconstruction, and
@@ -1834,28 +1836,28 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
         else
             recon(flux_y, vof, phi, k == 1, false, nullptr, nullptr);
         const SweepIn s1{vof, phi, B.fr, B.fl};
-        SG_HIP(sweep_mark(0));
+        if ((rc = sweep_mark(0))) return rc;
         if (k % 2 == 1)
             hipLaunchKernelGGL((k_sweep<true, true>), sgrd, sblk, 0, st, G, s1, bits, dtv, open, nullptr, B.tv, B.vt,
                                B.pt);
         else
             hipLaunchKernelGGL((k_sweep<false, true>), sgrd, sblk, 0, st, G, s1, bits, dtv, open, nullptr, B.tv, B.vt,
                                B.pt);
-        SG_HIP(sweep_mark(1));
+        if ((rc = sweep_mark(1))) return rc;
         // second sweep: (vt, pt) -> (vof, phi), explicit divergence
         if (k % 2 == 1)
             recon(flux_y, B.vt, B.pt, false, false, nullptr, nullptr);
         else
             recon(flux_x, B.vt, B.pt, false, false, nullptr, nullptr);
         const SweepIn s2{B.vt, B.pt, B.fr, B.fl};
-        SG_HIP(sweep_mark(0));
+        if ((rc = sweep_mark(0))) return rc;
         if (k % 2 == 1)
             hipLaunchKernelGGL((k_sweep<false, false>), sgrd, sblk, 0, st, G, s2, bits, dtv, open, B.tv, nullptr, vof,
                                phi);
         else
             hipLaunchKernelGGL((k_sweep<true, false>), sgrd, sblk, 0, st, G, s2, bits, dtv, open, B.tv, nullptr, vof,
                                phi);
-        SG_HIP(sweep_mark(1));
+        if ((rc = sweep_mark(1))) return rc;
         if (moves) {
             // ObjectMovement (Clsvof_Mod.f90:2384-2398) over the sub-step,
             // then SolidVolumeFraction on the P cells (:920-921)
@@ -1864,8 +1866,7 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
             m.shape.cx = m.shape.cx + 0.5 * m.asx * (dtv * dtv) + m.us * dtv;
             m.us = m.us + m.asx * dtv;
             m.vs = m.vs + m.asy * dtv;
-            const int rc = solid_fraction_step(c, &m.shape);
-            if (rc) return rc;
+            if ((rc = solid_fraction_step(c, &m.shape))) return rc;
             // the solid has changed vof too
             hipLaunchKernelGGL(k_bc, rgrd, rblk, 0, st, c->ni, c->nj, vof, phi);
         }
