@@ -211,7 +211,7 @@ int sg_interface_to_uv_resident(sg_ctx* ctx);
  * (the geometry of sg_set_geometry plus the solid line NXS/NYS/PHIS).
  * Needs ni, nj >= 4. */
 typedef struct sg_clsvof_params {
-    int nsub; /* sub-steps per call (nv = 6, Clsvof_Mod.f90:754) */
+    int nsub; /* sub-steps per call, 1 to 1024 (nv = 6, Clsvof_Mod.f90:754) */
     /* west inflow of X_Sweep (:1057-1059): row j takes in liquid through its
      * west face while y_j - dy_j/2 < depth + amp*sin(kw*xw - omega*(time +
      * k*dt/nsub)) at sub-step k, xw the west edge of the grid

@@ -755,8 +755,8 @@ int sg_clsvof_advect_resident(sg_ctx* ctx, double dt, double time, const sg_clsv
         set_error("sg_clsvof_advect: the transport needs ni, nj >= 4");
         return SG_ERR_ARG;
     }
-    if (p->nsub < 1 || p->nsub > 1024) {
-        set_error("sg_clsvof_advect: nsub must be in [1, 1024]");
+    if (p->nsub < 1 || p->nsub > ClsBuffers::MAX_NSUB) {
+        set_error("sg_clsvof_advect: nsub must be in [1, " + std::to_string(ClsBuffers::MAX_NSUB) + "]");
         return SG_ERR_ARG;
     }
     if (!(dt >= 0.0)) {

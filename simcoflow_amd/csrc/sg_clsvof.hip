@@ -1777,10 +1777,6 @@ int clsvof_advect(Ctx* c, double dt, int nsub) {
     const dim3 sblk(SWEEP_W, SWEEP_H), sgrd((c->ni + SWEEP_W - 1) / SWEEP_W, (c->nj + SWEEP_H - 1) / SWEEP_H);
     const double dtv = dt / (double)nsub;
     hipStream_t st = c->stream;
-    if (nsub > ClsBuffers::MAX_NSUB) {
-        set_error("clsvof_advect: too many sub-steps");
-        return SG_ERR_ARG;
-    }
     // the number of sources listed, one per sub-step
     hipLaunchKernelGGL(k_zero, dim3((nsub + 255) / 256), dim3(256), 0, st, B.cnt, nsub);
     Bits bits;

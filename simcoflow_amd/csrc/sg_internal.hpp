@@ -155,7 +155,7 @@ struct ClsBuffers {
     int* srcs = nullptr;               // listed interface cells (re-distancing sources)
     double* fr = nullptr;              // PLIC flux through the far / near face of a sweep, where a cell needs it
     double* fl = nullptr;
-    static constexpr int MAX_NSUB = 614;
+    static constexpr int MAX_NSUB = 1024;  // sub-steps a call
     unsigned* cnt = nullptr;           // sources listed, one count per sub-step
     unsigned long long* bits = nullptr;  // the cells' class bits, four planes of mw x nj words
     unsigned char* open = nullptr;     // sweep tiles free of solid

@@ -1,12 +1,13 @@
-"""The transport with many sub-steps a call: the sweep timer's pool of event pairs
-runs out within one."""
+"""The transport with many sub-steps a call: up to the most it takes, bit for bit
+against the CPU oracle as elsewhere, and refused beyond; the sweep timer's pool of
+event pairs runs out within one."""
 import ctypes
 
 import numpy as np
 import pytest
 
 from simcoflow_amd import cases as C
-from test_gpu_clsvof import _ctx
+from test_gpu_clsvof import _ctx, _run_both
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +35,22 @@ def test_sweep_timer_counts_every_sweep(nsub):
         pj.close()
     assert n.value == 4 * nsub and ms.value > 0.0
     assert np.isfinite(vof).all() and np.isfinite(phi).all()
+
+
+@pytest.mark.parametrize("nsub", [614, 615, 1024])
+def test_most_sub_steps_bit_exact(oracle_lib, nsub):
+    case, u, v = _case()
+    print(f"[clsvof] {nsub} sub-steps", flush=True)
+    _run_both(oracle_lib, case.grid, case.geo, case.itf.vof, case.itf.phi, u, v, case.dt, steps=1, nsub=nsub)
+
+
+@pytest.mark.parametrize("nsub", [-1, 0, 1025])
+def test_sub_steps_out_of_range_refused(nsub):
+    from simcoflow_amd import _lib
+    case, u, v = _case()
+    pj = _ctx(case.grid, case.geo)
+    try:
+        with pytest.raises(_lib.SimcoError, match=r"nsub must be in \[1, 1024\]"):
+            pj.clsvof_advect(case.itf.vof, case.itf.phi, u, v, case.dt, nsub=nsub)
+    finally:
+        pj.close()
