@@ -212,10 +212,11 @@ int sg_interface_to_uv_resident(sg_ctx* ctx);
  * Needs ni, nj >= 4. */
 typedef struct sg_clsvof_params {
     int nsub; /* sub-steps per call, 1 to 1024 (nv = 6, Clsvof_Mod.f90:754) */
-    /* west inflow of X_Sweep (:1057-1059): row j takes in liquid through its
-     * west face while y_j - dy_j/2 < depth + amp*sin(kw*xw - omega*(time +
-     * k*dt/nsub)) at sub-step k, xw the west edge of the grid
-     * (Depthw, Amp0, kw, omew of StateVariables.f90:24-25) */
+    /* Depthw, Amp0, kw, omew of StateVariables.f90:24-25, the west inflow wave of
+     * X_Sweep (:1057-1059).  Accepted, like the calls' `time`, so that a host can
+     * pass what the reference passes, and without effect: the inflow enters the
+     * cells of the domain's ring only, which Boundary_Condition (:961-973)
+     * overwrites with their inner neighbours before anything reads them. */
     double depth, amp, kw, omega;
 } sg_clsvof_params;
 
@@ -228,7 +229,7 @@ int sg_set_centres(sg_ctx* ctx, const double* xc, const double* yc);
 int sg_clsvof_advect_resident(sg_ctx* ctx, double dt, double time, const sg_clsvof_params* p);
 /* Drop-in body of Coupled_LS_VOF: host in/out.  vof/phi = PCell%vof/phi
  * (in/out), nx/ny = PCell%nx/ny (out, may be NULL), u/v = TVar%u/v
- * (ghosted), time = NondiT. */
+ * (ghosted), time = NondiT (without effect, see sg_clsvof_params). */
 int sg_clsvof_advect(sg_ctx* ctx, double* vof, double* phi, double* nx, double* ny, const double* u,
                      const double* v, double dt, double time, const sg_clsvof_params* p);
 

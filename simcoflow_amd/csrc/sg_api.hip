@@ -732,7 +732,7 @@ int sg_clsvof_params_default(sg_clsvof_params* p) {
     if (!p) return SG_ERR_ARG;
     std::memset(p, 0, sizeof(*p));
     p->nsub = 6;          // Clsvof_Mod.f90:754
-    p->depth = 1.0e300;   // inflow open on every row
+    p->depth = 1.0e300;   // inflow open on every row (no effect on the transport)
     return SG_OK;
 }
 

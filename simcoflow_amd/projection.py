@@ -180,6 +180,10 @@ class Projection:
 
     # -- interface transport -------------------------------------------------
     def clsvof_params(self, nsub=6, wave=None):
+        """wave: (depth, amp, kw, omega) of X_Sweep's west inflow
+        (Clsvof_Mod.f90:1057-1059); kept in the parameters, without effect on
+        the transport (nor has its time): the inflow only reaches ring cells,
+        which the boundary copy overwrites."""
         p = _lib.ClsvofParams()
         check(self.lib.sg_clsvof_params_default(ctypes.byref(p)))
         p.nsub = nsub
