@@ -18,6 +18,7 @@
 #include <algorithm>
 
 #include "sg_internal.hpp"
+#include "sg_divisor.hpp"
 
 namespace sg {
 
@@ -67,20 +68,6 @@ __device__ int locate(const double* __restrict__ c, const double* __restrict__ h
     }
     return -1;
 }
-
-// a / d, correctly rounded, for a d that many a share: r = 1 / d.  The product
-// a r is within two units in the last place, one correction makes it faithful
-// and the second, whose remainder is exact, rounds as the division does
-// (Markstein's theorem) while nothing leaves the normal range.
-struct Divisor {
-    double d, r;
-    __device__ explicit Divisor(double v) : d(v), r(1.0 / v) {}
-    __device__ static bool safe(double v) { return fabs(v) > 0x1p-60 && fabs(v) < 0x1p60; }
-    __device__ __forceinline__ double operator()(double a) const {
-        const double q = a * r, p = __builtin_fma(__builtin_fma(-d, q, a), r, q);
-        return __builtin_fma(__builtin_fma(-d, p, a), r, p);
-    }
-};
 
 // One sub-step's chain -- square root, quotients, pow, exp -- is the kernel's
 // time: with 1e5 particles there are one or two wavefronts a SIMD, and each
