@@ -145,6 +145,7 @@ int sg_ctx_create(int ni, int nj, const double* dx, const double* dy, const doub
     }
     Ctx* c = new Ctx();
     if (const char* ev = std::getenv("SG_NO_GRAPH")) c->use_graph = (ev[0] == '0');
+    if (const char* ev = std::getenv("SG_NO_FUSED_SUMS")) c->fuse_sums = (ev[0] == '0');
     c->ni = ni;
     c->nj = nj;
     c->prm = *prm;

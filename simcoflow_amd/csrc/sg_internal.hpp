@@ -292,6 +292,7 @@ struct Ctx {
         double ms = 0.0;
     } sweep_timing;
     int use_graph = 1;
+    int fuse_sums = 1;  // the PCG's kernels add up few partials themselves
     ClsBuffers cls;
     StagDev stag[2];  // U, V cells
     PredBuffers pred;

@@ -424,8 +424,8 @@ int enqueue_iteration_t(Ctx* c, int parity, V* r, V* z, V* q, V* p0, V* p1) {
     const int nb_pq = (int)(gd.x * gd.y);
     // without a deflation vector between them, the kernels that use (r,z) and
     // (p,q) add the partials up themselves where those are few enough
-    const bool defl = deflating(c);
-    const int sum_rz = !defl && nb_rz <= FUSE_MAX ? nb_rz : 0, sum_pq = !defl && nb_pq <= FUSE_MAX ? nb_pq : 0;
+    const bool defl = deflating(c), fuse = c->fuse_sums && !defl;
+    const int sum_rz = fuse && nb_rz <= FUSE_MAX ? nb_rz : 0, sum_pq = fuse && nb_pq <= FUSE_MAX ? nb_pq : 0;
     if (!sum_rz) hipLaunchKernelGGL(k_finalize, dim3(1), dim3(NTF), 0, s, S1, nb_rz, (int)FIN_RZ, c->sc, 0.0);
     const double* w = nullptr;
     if (defl) {

@@ -30,3 +30,21 @@ def test_sums_of_any_number_of_partials(oracle_lib, precision):
         its[partials] = info.iterations
     print(f"[pcg sums] iterations {its}", flush=True)
     assert abs(its[288] - its[256]) <= 2
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("ni,nj,partials", SIZES + [(7, 5, 1), (130, 16, 3), (448, 250, 112)])
+def test_sums_are_those_of_a_finalize_launch(monkeypatch, ni, nj, partials, precision):
+    """The same solve with the sums added up by the kernels that use them and by
+    launches of their own: the same iterations and the same pressure in every bit,
+    which any other order of a sum's terms would change."""
+    assert -(-ni // 64) * -(-nj // 16) == partials
+    print(f"[pcg sums] fused or not {ni}x{nj} {partials} partials precision {precision}", flush=True)
+    case = _case(ni, nj)
+    got = []
+    for off in ("0", "1"):
+        monkeypatch.setenv("SG_NO_FUSED_SUMS", off)
+        p, info, _, _ = _solve(case, precision, 4, tol=1e-9)
+        got.append((p, info.iterations, info.relres))
+    assert got[0][1:] == got[1][1:]
+    assert np.array_equal(got[0][0], got[1][0])
