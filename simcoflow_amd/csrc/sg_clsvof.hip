@@ -1752,11 +1752,13 @@ int sweep_timing_drain(Ctx* c) {
 }
 
 // From how many cells a call works out which of its sweep tiles are free of
-// solid.  Measured on a whole call of 6 sub-steps (12 sweeps) with and without:
-// at 2048^2, where a sweep is bound by its bytes, 1498 against 1612 us; at 1024^2,
-// 768^2 and 512^2, where its arrays stay in the last-level cache, 641 against 640,
-// 586 against 585 and 508 against 491 us.  Their 3 arrays of results and 3 of
-// operands outgrow that cache's 256 MB together with the geometry between the two.
+// solid.  A call of 6 sub-steps (12 sweeps) and the U/V interface with and without,
+// us, a swarm of bubbles: 724^2 642 / 641, 1024^2 798 / 792, 1200^2 906 / 924, 1448^2
+// 1063 / 1134, 1600^2 1200 / 1311, 1800^2 1440 / 1606, 2048^2 1835 / 1960; waves with a
+// solid 4096 x 2048 3150 / 3318; the sweeps alone at 512^2 508 / 491.  The flags pay
+// for themselves from about 1.2 million cells, where a sweep's arrays, 104 bytes a
+// cell with the geometry, are half the last-level cache's 256 MB and other kernels'
+// take the rest; the line stands where they gain 6%, not where they break even.
 constexpr size_t OPEN_MIN_CELLS = 1ull << 21;
 
 // Coupled_LS_VOF on the device fields VOF, PHI (in/out), NX, NY (out),
