@@ -292,9 +292,8 @@ __device__ inline void raw_fce(const GridSpec& G, const GeoOut& o, int gi, int j
 // face centres follow :91-117 (the rows of FCN copy FCE).
 //
 // Three grids of 1024 x 512 take 43.5 us (52.4 in three launches, which a closing
-// pass and a copy followed for U and V).  Its 8 arrays of results are 100 MB, half
-// of that at the rate of a copy: the rest is the edges' chains of divisions, each
-// worked out again by the cells on its other side.
+// pass and a copy followed for U and V).  Bound by bytes, reads and writes alike: at
+// 2048^2 the counters read 0.73 GB and 0.83 GB written in 0.46 ms, 3.4 TB/s.
 __global__ void __launch_bounds__(256) k_geo_faces(Grids A) {
 #pragma clang fp contract(off)
     const GridSpec& G = A.G[blockIdx.z];
